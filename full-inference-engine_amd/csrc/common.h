@@ -358,6 +358,65 @@ FIE_DEV uint64_t dwave_sum_u64(uint64_t v)
     return t;
 }
 
+FIE_DEV uint64_t dwave_max_u64(uint64_t v)
+{
+    auto step = [](uint64_t x, auto mv) {
+        const uint64_t o = ((uint64_t)mv((uint32_t)(x >> 32)) << 32) | mv((uint32_t)x);
+        return o > x ? o : x;
+    };
+    v = step(v, [](uint32_t a) { return dpp_mov<kDppXor1>(a); });
+    v = step(v, [](uint32_t a) { return dpp_mov<kDppXor2>(a); });
+    v = step(v, [](uint32_t a) { return dpp_mov<kDppHalfMirror>(a); });
+    v = step(v, [](uint32_t a) { return dpp_mov<kDppMirror>(a); });
+    uint64_t t = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const uint64_t o = ((uint64_t)rl((uint32_t)(v >> 32), 16 * r) << 32) | rl((uint32_t)v, 16 * r);
+        t = o > t ? o : t;
+    }
+    return t;
+}
+
+FIE_DEV uint32_t dwave_sum_u32(uint32_t v)
+{
+    v += dpp_mov<kDppXor1>(v);
+    v += dpp_mov<kDppXor2>(v);
+    v += dpp_mov<kDppHalfMirror>(v);
+    v += dpp_mov<kDppMirror>(v);
+    return rl(v, 0) + rl(v, 16) + rl(v, 32) + rl(v, 48);
+}
+
+// Sum of values below 2^116 (masses are below 2^104): two limbs of at most 58 bits,
+// whose wave sums fit 64.
+FIE_DEV u128 dwave_sum_u128(u128 v)
+{
+    constexpr uint64_t kLimb = (1ull << 58) - 1;
+    return ((u128)dwave_sum_u64((uint64_t)(v >> 58)) << 58) + dwave_sum_u64((uint64_t)v & kLimb);
+}
+
+// Inclusive prefix sum over the lanes of a wave (lane 0 first).
+FIE_DEV uint64_t dwave_incl_scan_u64(uint64_t v)
+{
+    const int row = (threadIdx.x & 63) >> 4;
+    // inside each row of 16: shifts by 1, 2, 4, 8 (0 shifted in)
+    auto step = [](uint64_t x, auto mv) { return x + (((uint64_t)mv((uint32_t)(x >> 32)) << 32) | mv((uint32_t)x)); };
+#define FIE_SHR(N) [](uint32_t a) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)a, 0x110 | N, 0xF, 0xF, true); }
+    v = step(v, FIE_SHR(1));
+    v = step(v, FIE_SHR(2));
+    v = step(v, FIE_SHR(4));
+    v = step(v, FIE_SHR(8));
+#undef FIE_SHR
+    auto at = [&](int lane) { return ((uint64_t)rl((uint32_t)(v >> 32), lane) << 32) | rl((uint32_t)v, lane); };
+    const uint64_t r0 = at(15), r1 = at(31), r2 = at(47);
+    return v + (row > 0 ? r0 : 0) + (row > 1 ? r1 : 0) + (row > 2 ? r2 : 0);
+}
+
+FIE_DEV u128 dwave_incl_scan_u128(u128 v)
+{
+    constexpr uint64_t kLimb = (1ull << 58) - 1;
+    return ((u128)dwave_incl_scan_u64((uint64_t)(v >> 58)) << 58) + dwave_incl_scan_u64((uint64_t)v & kLimb);
+}
+
 // Exclusive prefix sum over the lanes of a wave (lane 0 first), and the total.
 FIE_DEV uint32_t dwave_excl_scan_u32(uint32_t v, uint32_t* total)
 {
@@ -451,7 +510,7 @@ FIE_DEV uint64_t block_sum_u64(uint64_t v, uint64_t* scratch)
 template <int NT>
 FIE_DEV u128 block_sum_u128(u128 v, u128* scratch)
 {
-    v = wave_sum_u128(v);
+    v = dwave_sum_u128(v);
     if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
     __syncthreads();
     u128 t = 0;

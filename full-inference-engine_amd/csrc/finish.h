@@ -34,15 +34,32 @@ struct SelResult {
     int found;
 };
 
+// One window of the windowed full-row path (window.h).
+struct Win {
+    uint64_t lo, hi;     // packed composites, inclusive
+    float above;         // estimated mass above it, in units of the row maximum's weight
+    float yh;            // the value of its one key (byidx)
+    uint32_t n;          // tokens counted in it
+    uint32_t kmin, kmax; // the keys a refining count met
+    int byidx, split;    // refined by index (it may hold one key only); it held several
+    int sh;              // shift of its finer bins
+};
+
 struct FinSmem {
     uint64_t cand[kGCap];                       // candidates or a gathered key range
-    uint32_t pc[kPassBins];                     // full-row pass: counts per bin
     union {
-        uint64_t pm_lo[kPassBins];              // full-row pass: mass per bin (low limb)
-        float pmf[kPassBins];                   // candidate narrowing: float mass per bin
+        struct {
+            uint32_t pc[kPassBins];             // full-row pass: counts per bin
+            uint64_t pm_lo[kPassBins];          // mass per bin: its low limb (full-row pass), or in
+                                                // units of 2^-31 of the maximum's (narrowing)
+            uint64_t pm_hi[kPassBins];          // full-row pass: mass per bin (high limb)
+            uint32_t cnt[kChunk];               // penalty counts of one chunk
+        };
+        struct {                                // windowed passes: a wave's tile
+            uint32_t cnt[kFinThreads / 64][kTile / 2];   // its penalty counts (u16 halves)
+            uint32_t bits[kFinThreads / 64][kTile / 32]; // its penalised tokens
+        } tp;
     };
-    uint64_t pm_hi[kPassBins];                  // full-row pass: mass per bin (high limb)
-    uint32_t cnt[kChunk];                       // penalty counts of one chunk
     uint32_t snb[kMaxSpans];                    // history ids per span (k_prep), of a pass's row
     uint32_t hc[256];                           // LDS selection: counts per digit
     uint64_t hm_lo[256], hm_hi[256];            // LDS selection: mass per digit
@@ -58,6 +75,10 @@ struct FinSmem {
     u128 bex, bme;
     uint32_t bcnt;
     uint64_t cmax;
+    Win win[2];                                 // windowed path: its windows,
+    int wjl, wjh;                               // a pick's bins and their counts,
+    uint32_t wcl, wch, wn, wbig;                // tokens gathered, windows to refine
+    float wab;
     SelResult sel;
     DeferRec dfr;                               // a row deferred to the full-row path in place
     uint32_t dmode;                             // its mode (0: not deferred)
@@ -107,7 +128,7 @@ struct Pred {
 // MASS) first exceeds g: excl <= g < excl + meas.  Digits are 8-bit windows placed
 // just below the common prefix of the remaining range, so few levels are needed.
 template <bool MASS>
-FIE_DEV SelResult lds_select(FinSmem& S, int n, const Pred pr, u128 g)
+FIE_DEV SelResult lds_select(FinSmem& S, const uint64_t* cand, int n, const Pred pr, u128 g)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint64_t prefix = 0, pmask = 0;
@@ -116,7 +137,7 @@ FIE_DEV SelResult lds_select(FinSmem& S, int n, const Pred pr, u128 g)
         // range of the remaining elements (one barrier), and a cleared histogram
         uint64_t mn = ~0ull, mx = 0;
         for (int i = tid; i < n; i += kFinThreads) {
-            const uint64_t c = S.cand[i];
+            const uint64_t c = cand[i];
             if ((c & pmask) == prefix && pr(c)) {
                 mn = c < mn ? c : mn;
                 mx = c > mx ? c : mx;
@@ -126,8 +147,8 @@ FIE_DEV SelResult lds_select(FinSmem& S, int n, const Pred pr, u128 g)
             S.hc[i] = 0;
             if (MASS) { S.hm_lo[i] = 0; S.hm_hi[i] = 0; }
         }
-        mx = wave_max_u64(mx);
-        mn = ~wave_max_u64(~mn);
+        mx = dwave_max_u64(mx);
+        mn = ~dwave_max_u64(~mn);
         if (lane == 0) { S.red64[wave] = mx; S.red64[8 + wave] = mn; }
         __syncthreads();
         mx = 0;
@@ -147,7 +168,7 @@ FIE_DEV SelResult lds_select(FinSmem& S, int n, const Pred pr, u128 g)
         const int shift = hb >= 7 ? hb - 7 : 0;
         const uint64_t hmask = (hb >= 63) ? 0ull : ~((2ull << hb) - 1);
         for (int i = tid; i < n; i += kFinThreads) {
-            const uint64_t c = S.cand[i];
+            const uint64_t c = cand[i];
             if ((c & pmask) == prefix && pr(c)) {
                 const int d = (int)((c >> shift) & 0xFFu);
                 if (MASS) {
@@ -172,7 +193,7 @@ FIE_DEV SelResult lds_select(FinSmem& S, int n, const Pred pr, u128 g)
                 loc[q] = MASS ? (((u128)S.hm_hi[d] << 64) | S.hm_lo[d]) : (u128)S.hc[d];
                 sum += loc[q];
             }
-            const u128 incl = wave_incl_scan_u128(sum);
+            const u128 incl = dwave_incl_scan_u128(sum);
             u128 run = incl - sum;
             if (run <= g && g < incl) {
 #pragma unroll
@@ -204,14 +225,11 @@ FIE_DEV SelResult lds_select(FinSmem& S, int n, const Pred pr, u128 g)
 // ---------------------------------------------------------------- full-row passes
 // Visit every token of the row once, re-reading it from memory: f(y, idx) with each
 // token's scaled (penalised) logit, token 0 with its settled value.  The row streams
-// in kChunk-token chunks through a ring of kPassDepth register buffers, the next
-// chunks' loads in flight while one is processed.  A pass is bound by its per-token
-// instructions: the third buffer gains 3% on many full-row rows at once and nothing
-// on a single one.  A penalised row's counts come
-// from k_prep's span bucket, loaded with the chunk (one id per thread: kBucketCap ==
-// kFinThreads), so counting never waits on a dependent load; a span whose bucket
-// overflowed is counted from the whole history instead.
-constexpr int kPassDepth = 3;
+// in kChunk-token chunks, the next chunk's loads in flight while one is processed.
+// Rows get here seldom (top-k or min-p thresholds below the candidates), so the loop
+// is kept small.  A penalised row's counts come from k_prep's span bucket, loaded with
+// the chunk (one id per thread: kBucketCap == kFinThreads), so counting never waits on
+// a dependent load; a span whose bucket overflowed is counted from the whole history.
 static_assert(kBucketCap == kFinThreads && kSpan == 2 * kChunk, "bucket entries per thread, chunks per span");
 
 template <int DT, bool VEC, class F>
@@ -220,152 +238,72 @@ FIE_DEV void row_pass(FinSmem& S, const KParams& P, int row, float s, bool pen, 
 {
     constexpr int EPL = DTy<DT>::EPL, SZ = DTy<DT>::SZ;
     constexpr int NL = kChunk / kFinThreads / EPL;
-    constexpr int D = kPassDepth;
     const fie_sampler_args& a = P.a;
     const int V = a.vocab, tid = threadIdx.x;
-    const int nch = (V + kChunk - 1) / kChunk;
     const char* rowp = (const char*)a.logits + (size_t)row * (size_t)a.row_stride * SZ;
     const bool mark = s != 1.0f && s >= 0x1p-30f && s <= 0x1p30f;
     const float rs = 1.0f / s;
     if (tid == 0 && k0) f(key_to_float(k0), 0u);
-    uint4 buf[D][NL];
-    uint32_t bof[D];
-    bool overflow = false;
+    uint4 nxt[NL];
+    uint32_t nof = 0;
     if (pen) {
-        for (int i = tid; i < P.NS; i += kFinThreads) {
-            const uint32_t nb = P.w.nb[(size_t)row * P.NS + i];
-            S.snb[i] = nb;
-            overflow |= nb > (uint32_t)kBucketCap;
-        }
+        for (int i = tid; i < P.NS; i += kFinThreads) S.snb[i] = P.w.nb[(size_t)row * P.NS + i];
+        __syncthreads();
     }
-    if (VEC && !__syncthreads_or(overflow)) {
-        // The common case, as straight-line streaming: whole chunks, one vector load
-        // per group, every span's bucket complete.  Every step of the ring issues the
-        // same loads (past the last whole chunk it reloads that chunk, unused), so the
-        // compiler's wait counts see the D - 1 chunks still in flight; the partial
-        // last chunk follows the ring.
-        const int nfull = V / kChunk;
-        auto issue_full = [&](uint4 (&b)[NL], uint32_t& of, int c) {
-            const int lo = (c < nfull ? c : nfull - 1) * kChunk;
+    auto issue = [&](int lo) {
 #pragma unroll
-            for (int j = 0; j < NL; ++j) b[j] = *(const uint4*)(rowp + (size_t)(lo + (j * kFinThreads + tid) * EPL) * SZ);
-            of = P.w.bk[((size_t)row * P.NS + lo / kSpan) * kBucketCap + tid];
-        };
-        auto count_bucket = [&](uint32_t of, int lo) {
+        for (int j = 0; j < NL; ++j) nxt[j] = load_group<DT, VEC>(rowp, lo + (j * kFinThreads + tid) * EPL, V);
+        if (pen) {
+            // a chunk past the row's end reads the last span's entry, unused
+            const int sp = lo / kSpan < P.NS ? lo / kSpan : P.NS - 1;
+            nof = P.w.bk[((size_t)row * P.NS + sp) * kBucketCap + tid];
+        }
+    };
+    issue(0);
+#pragma unroll 1
+    for (int lo = 0; lo < V; lo += kChunk) {
+        uint4 cur[NL];
+#pragma unroll
+        for (int j = 0; j < NL; ++j) cur[j] = nxt[j];
+        const uint32_t of = nof;
+        issue(lo + kChunk);
+        if (pen) {
             for (int i = tid; i < kChunk / 4; i += kFinThreads) ((uint4*)S.cnt)[i] = make_uint4(0, 0, 0, 0);
             __syncthreads();
-            const uint32_t o = of - (uint32_t)(lo % kSpan);
-            if ((uint32_t)tid < S.snb[lo / kSpan] && o < (uint32_t)kChunk) atomicAdd(&S.cnt[o], 1u);
+            const uint32_t nb = S.snb[lo / kSpan];
+            if (nb <= (uint32_t)kBucketCap) {
+                const uint32_t o = of - (uint32_t)(lo % kSpan);
+                if ((uint32_t)tid < nb && o < (uint32_t)kChunk) atomicAdd(&S.cnt[o], 1u);
+            } else {
+                const int hi = min(lo + kChunk, V);
+                const int64_t h0 = a.hist_offsets[row], h1 = hist_end(a, row);
+                for (int64_t h = h0 + tid; h < h1; h += kFinThreads) {
+                    const uint32_t id = (uint32_t)a.hist_ids[h];
+                    if (id >= (uint32_t)lo && id < (uint32_t)hi && id != 0) atomicAdd(&S.cnt[id - lo], 1u);
+                }
+            }
             __syncthreads();
-        };
-        auto visit = [&](const uint4 (&b)[NL], int lo) {
+        }
 #pragma unroll
-            for (int j = 0; j < NL; ++j) {
-                const int e0 = lo + (j * kFinThreads + tid) * EPL;
+        for (int j = 0; j < NL; ++j) {
+            const int e0 = lo + (j * kFinThreads + tid) * EPL;
 #pragma unroll
-                for (int e = 0; e < EPL; ++e) {
-                    const int idx = e0 + e;
-                    if (idx >= V || idx == 0) continue;
-                    float x = lane_get<DT>(b[j], e);
-                    if (pen) {
-                        const uint32_t cc = S.cnt[idx - lo];
-                        if (cc) x = penalize(x, rep, pres, freq, cc);
-                    }
-                    float y;
-                    if (s == 1.0f) y = x + 0.0f;
-                    else if (mark && markstein_ok(x)) y = div_markstein(x, s, rs) + 0.0f;
-                    else y = scaled(x, s);
-                    f(y, (uint32_t)idx);
+            for (int e = 0; e < EPL; ++e) {
+                const int idx = e0 + e;
+                if (idx >= V || idx == 0) continue;
+                float x = lane_get<DT>(cur[j], e);
+                if (pen) {
+                    const uint32_t cc = S.cnt[idx - lo];
+                    if (cc) x = penalize(x, rep, pres, freq, cc);
                 }
-            }
-        };
-        if (nfull > 0) {
-#pragma unroll
-            for (int q = 0; q < D; ++q) issue_full(buf[q], bof[q], q);
-            for (int c0 = 0; c0 < nfull; c0 += D) {
-#pragma unroll
-                for (int q = 0; q < D; ++q) {
-                    const int c = c0 + q;
-                    if (c < nfull) {
-                        if (pen) count_bucket(bof[q], c * kChunk);
-                        visit(buf[q], c * kChunk);
-                        if (pen) __syncthreads();
-                    }
-                    issue_full(buf[q], bof[q], c + D);
-                }
+                float y;
+                if (s == 1.0f) y = x + 0.0f;
+                else if (mark && markstein_ok(x)) y = div_markstein(x, s, rs) + 0.0f;
+                else y = scaled(x, s);
+                f(y, (uint32_t)idx);
             }
         }
-        const int lo = nfull * kChunk;
-        if (lo < V) {
-#pragma unroll
-            for (int j = 0; j < NL; ++j) buf[0][j] = load_group<DT, VEC>(rowp, lo + (j * kFinThreads + tid) * EPL, V);
-            if (pen) count_bucket(P.w.bk[((size_t)row * P.NS + lo / kSpan) * kBucketCap + tid], lo);
-            visit(buf[0], lo);
-        }
-        __syncthreads();
-        return;
-    }
-    auto issue = [&](uint4 (&b)[NL], uint32_t& of, int c) {
-        const int lo = c * kChunk;
-#pragma unroll
-        for (int j = 0; j < NL; ++j) b[j] = load_group<DT, VEC>(rowp, lo + (j * kFinThreads + tid) * EPL, V);
-        if (pen) {
-            // a chunk past the row's end (the ring's tail) reads the last span's entry, unused
-            const int sp = lo / kSpan < P.NS ? lo / kSpan : P.NS - 1;
-            of = P.w.bk[((size_t)row * P.NS + sp) * kBucketCap + tid];
-        }
-    };
-    auto count = [&](uint32_t of, int lo, int hi) {
-        if (lo >= V) return;                                     // uniform: no token to count
-        for (int i = tid; i < kChunk / 4; i += kFinThreads) ((uint4*)S.cnt)[i] = make_uint4(0, 0, 0, 0);
-        __syncthreads();
-        const uint32_t nb = S.snb[lo / kSpan];
-        if (nb <= (uint32_t)kBucketCap) {
-            const uint32_t o = of - (uint32_t)(lo % kSpan);
-            if ((uint32_t)tid < nb && o < (uint32_t)kChunk) atomicAdd(&S.cnt[o], 1u);
-        } else {
-            const int64_t h0 = a.hist_offsets[row], h1 = hist_end(a, row);
-            for (int64_t h = h0 + tid; h < h1; h += kFinThreads) {
-                const uint32_t id = (uint32_t)a.hist_ids[h];
-                if (id >= (uint32_t)lo && id < (uint32_t)hi && id != 0) atomicAdd(&S.cnt[id - lo], 1u);
-            }
-        }
-        __syncthreads();
-    };
-#pragma unroll
-    for (int q = 0; q < D; ++q)
-        if (q < nch) issue(buf[q], bof[q], q);
-    // a ring of D buffers in fixed roles (no register copies, which would wait on
-    // loads still in flight): buffer q holds chunk c0 + q while the others load.
-    // Past the row's end the loads read nothing and every token fails idx < V.
-    for (int c0 = 0; c0 < nch; c0 += D) {
-#pragma unroll
-        for (int q = 0; q < D; ++q) {
-            const int c = c0 + q;
-            const int lo = c * kChunk, hi = min(lo + kChunk, V);
-            if (pen) count(bof[q], lo, hi);
-#pragma unroll
-            for (int j = 0; j < NL; ++j) {
-                const int e0 = lo + (j * kFinThreads + tid) * EPL;
-#pragma unroll
-                for (int e = 0; e < EPL; ++e) {
-                    const int idx = e0 + e;
-                    if (idx >= V || idx == 0) continue;
-                    float x = lane_get<DT>(buf[q][j], e);
-                    if (pen) {
-                        const uint32_t cc = S.cnt[idx - lo];
-                        if (cc) x = penalize(x, rep, pres, freq, cc);
-                    }
-                    float y;
-                    if (s == 1.0f) y = x + 0.0f;
-                    else if (mark && markstein_ok(x)) y = div_markstein(x, s, rs) + 0.0f;
-                    else y = scaled(x, s);
-                    f(y, (uint32_t)idx);
-                }
-            }
-            if (pen) __syncthreads();
-            issue(buf[q], bof[q], c + D);
-        }
+        if (pen) __syncthreads();
     }
     __syncthreads();
 }
@@ -416,7 +354,7 @@ FIE_DEV int pass_pick(FinSmem& S, int nbins, u128 g)
     }
     // block exclusive scan of u128 in thread order
     const int lane = tid & 63, wave = tid >> 6;
-    const u128 incl = wave_incl_scan_u128(sum);
+    const u128 incl = dwave_incl_scan_u128(sum);
     if (lane == 63) S.red128[wave] = incl;
     if (tid == 0) S.ibin = -1;
     __syncthreads();
@@ -494,7 +432,7 @@ FIE_DEV SelResult row_select(FinSmem& S, const KParams& P, int row, float s, boo
         if (cnt <= (uint32_t)kGCap) {
             const int n = pass_gather<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, pr,
                                                dg.shift, hiprefix);
-            SelResult r = lds_select<MASS>(S, n, pr, g);
+            SelResult r = lds_select<MASS>(S, S.cand, n, pr, g);
             r.excl += excl;
             return r;
         }
@@ -576,7 +514,7 @@ FIE_DEV int dbin_pick(FinSmem& S, int bmax, u128 last, u128 g, u128* above)
     u128 sum = 0;
 #pragma unroll
     for (int q = 0; q < per; ++q) sum += meas(tid * per + q);
-    const u128 incl = wave_incl_scan_u128(sum);
+    const u128 incl = dwave_incl_scan_u128(sum);
     if (lane == 63) S.red128[wave] = incl;
     if (tid == 0) S.ibin = -1;
     __syncthreads();
@@ -764,7 +702,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
         u128 above;
         const int b = dbin_pick<false>(S, kPassBins - 1, (u128)S.pc[kPassBins - 1], (u128)(topk - 1), &above);
         if (b < 0 || !gather(b, b)) return false;
-        const SelResult r = lds_select<false>(S, ncur, Pred{0, 0, 0}, (u128)(topk - 1) - above);
+        const SelResult r = lds_select<false>(S, S.cand, ncur, Pred{0, 0, 0}, (u128)(topk - 1) - above);
         if (!r.found) return false;
         tk = comp_k(r.comp);
     }
@@ -818,7 +756,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
                 uint64_t mn = ~0ull;
                 for (int i = tid; i < ncur; i += kFinThreads)
                     if (dbin_key(M, comp_k(S.cand[i])) < b) mn = S.cand[i] < mn ? S.cand[i] : mn;
-                mn = ~wave_max_u64(~mn);
+                mn = ~dwave_max_u64(~mn);
                 if ((tid & 63) == 0) S.red64[tid >> 6] = mn;
                 __syncthreads();
                 for (int w = 0; w < kFinThreads / 64; ++w) mn = S.red64[w] < mn ? S.red64[w] : mn;
@@ -827,7 +765,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
             }
             Pred pc{tau, 0, 0};
             pc.hi = chi;
-            const SelResult r = lds_select<true>(S, ncur, pc, thr - 1 - above);
+            const SelResult r = lds_select<true>(S, S.cand, ncur, pc, thr - 1 - above);
             if (!r.found) return false;
             cut = r.comp;
             T = above + r.excl + r.meas;
@@ -842,7 +780,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
         u128 above;
         const int b = dbin_pick<false>(S, kPassBins - 1, (u128)S.pc[kPassBins - 1], 0, &above);
         if (b < 0 || !gather(b, b)) return false;
-        const SelResult r = lds_select<false>(S, ncur, Pred{0, 0, 0}, 0);
+        const SelResult r = lds_select<false>(S, S.cand, ncur, Pred{0, 0, 0}, 0);
         if (!r.found) return false;
         tok = r.comp;
     } else {
@@ -861,7 +799,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
                 uint64_t mn = ~0ull;
                 for (int i = tid; i < ncur; i += kFinThreads)
                     if (dbin_key(M, comp_k(S.cand[i])) < b) mn = S.cand[i] < mn ? S.cand[i] : mn;
-                mn = ~wave_max_u64(~mn);
+                mn = ~dwave_max_u64(~mn);
                 if ((tid & 63) == 0) S.red64[tid >> 6] = mn;
                 __syncthreads();
                 for (int w = 0; w < kFinThreads / 64; ++w) mn = S.red64[w] < mn ? S.red64[w] : mn;
@@ -869,7 +807,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
                 pd.hi = mn - 1;
             }
         }
-        const SelResult r = lds_select<true>(S, ncur, pd, g - base);
+        const SelResult r = lds_select<true>(S, S.cand, ncur, pd, g - base);
         if (!r.found) return false;
         tok = r.comp;
     }
@@ -880,6 +818,23 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
     *tok_out = tok;
     return true;
 }
+
+FIE_DEV float wave_incl_scan_f32(float v)
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const float u = __shfl_up(v, d, 64);
+        if (lane >= d) v += u;
+    }
+    return v;
+}
+
+}  // namespace fie
+
+#include "window.h"
+
+namespace fie {
 
 // The shortest R2 prefix of the complete candidates S.cand[0, nv) holding at least
 // `cnt` elements and, when use_mass, mass above g, moved to S.cand[0, m); returns m
@@ -971,9 +926,11 @@ constexpr int kReloadQ = 5;
 static_assert(kCapW == 64, "one tile's candidate slots per wave");
 static_assert(kMaxTiles < kFinThreads, "the last thread is free for token 0");
 
-// Float mass of a token y relative to the row maximum M: rule R1's weight / 2^80 up
-// to the floors of R1 and the exponentials' rounding (used only to narrow).
-FIE_DEV float approx_mass(float y, float M) { return __expf(y - M); }
+// Mass of a token y relative to the row maximum M in units of 2^-31: rule R1's weight
+// / 2^49 up to the floors of R1, the exponentials' rounding and the truncation here
+// (used only to narrow).  Whole numbers, because an LDS atomic on floats takes 185
+// cycles a wave where one on 64-bit integers takes 21 (random bins, measured).
+FIE_DEV uint64_t approx_mass(float y, float M) { return (uint64_t)(uint32_t)(__expf(y - M) * 0x1p31f); }
 
 // The x-domain candidate slot as a y-domain composite.  rs = 1/s when s lies in
 // Markstein's range (cand_rs), else 0: inside the range the corrected product is
@@ -1022,17 +979,17 @@ FIE_DEV void cand_commit(FinSmem& S, const uint64_t (&cv)[Q], const bool (&ok)[Q
             const float y = key_to_float(comp_k(cv[q]));
             const int b = dbin_y(M, y);
             atomicAdd(&S.pc[b], 1u);
-            atomicAdd(&S.pmf[b], approx_mass(y, M));
+            atomicAdd((unsigned long long*)&S.pm_lo[b], (unsigned long long)approx_mass(y, M));
         }
     }
 }
 
 // The first sweep of a two-sweep commit: the held composites above `safe` are
-// counted (S.n, one LDS atomic per wave) and binned by d-bin (count, and float mass
-// when `mass`), the largest tracked; nothing is stored.  Called by whole waves.
+// counted (S.n, one LDS atomic per wave) and by d-bin, the largest tracked; nothing is
+// stored.  Called by whole waves.
 template <int Q>
 FIE_DEV void cand_count(FinSmem& S, const uint64_t (&cv)[Q], const bool (&ok)[Q], uint32_t safe,
-                        uint64_t& best, bool mass, float M)
+                        uint64_t& best, float M)
 {
     uint32_t k = 0;
 #pragma unroll
@@ -1041,13 +998,10 @@ FIE_DEV void cand_count(FinSmem& S, const uint64_t (&cv)[Q], const bool (&ok)[Q]
         best = cv[q] > best ? cv[q] : best;
         if (comp_k(cv[q]) > safe) {
             ++k;
-            const float y = key_to_float(comp_k(cv[q]));
-            const int b = dbin_y(M, y);
-            atomicAdd(&S.pc[b], 1u);
-            if (mass) atomicAdd(&S.pmf[b], approx_mass(y, M));
+            atomicAdd(&S.pc[dbin_key(M, comp_k(cv[q]))], 1u);
         }
     }
-    const uint32_t wk = wave_sum_u32(k);
+    const uint32_t wk = dwave_sum_u32(k);
     if ((threadIdx.x & 63) == 0 && wk) atomicAdd(&S.n, wk);
 }
 
@@ -1086,7 +1040,7 @@ FIE_DEV int load_candidates(FinSmem& S, const KParams& P, int row, int NT, float
     uint64_t best = 0;
     for (int t0 = 0; t0 < NT; t0 += kFinWaves * kReloadQ)
         cand_batch<kReloadQ>(S, P, row, NT, t0, s, safe, best, false, 0.0f, t0 == 0, comp_key(k0, 0));
-    best = wave_max_u64(best);
+    best = dwave_max_u64(best);
     if ((tid & 63) == 0 && best) atomicMax((unsigned long long*)&S.cmax, (unsigned long long)best);
     __syncthreads();
     const int m = (int)S.n;
@@ -1094,25 +1048,15 @@ FIE_DEV int load_candidates(FinSmem& S, const KParams& P, int row, int NT, float
     return m;
 }
 
-FIE_DEV float wave_incl_scan_f32(float v)
-{
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const float u = __shfl_up(v, d, 64);
-        if (lane >= d) v += u;
-    }
-    return v;
-}
-
 // narrow_candidates for a row binned as its candidates were taken (S.pc counts,
-// S.pmf float masses): the count criterion is exact; the mass criterion asks the
-// float prefix to exceed g by a margin (2^-9 relative, 2^-26 absolute, in units of
-// 2^80) that covers the float sums' rounding and the floors of rule R1, so the
+// S.pm_lo masses): the count criterion is exact; the mass criterion asks the
+// float prefix to exceed g by a margin (2^-9 relative, 2^-18 absolute, in units of
+// 2^80) that covers the float sums' rounding, the floors of rule R1 and 4096
+// candidates' truncation to 2^-31, so the
 // prefix it picks holds exact mass above g.  Should a crossing still fall past the
 // prefix, the exact selection finds no element there and reloads every candidate.
 // The last d-bin a narrowed prefix must keep, from the bins' counts (S.pc) and,
-// with use_mass, float masses (S.pmf): the bin where the running count reaches
+// with use_mass, masses (S.pm_lo): the bin where the running count reaches
 // cnt (cnt > 0) and the bin where the float prefix first exceeds g by the margin
 // described above, the later of the two; -1 when either is not found
 // (no narrowing).
@@ -1120,13 +1064,13 @@ FIE_DEV int binned_bound(FinSmem& S, int cnt, bool use_mass, u128 g)
 {
     constexpr int per = kPassBins / kFinThreads;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const float target = (float)(u128_to_double(g) * 0x1p-80 * (1.0 + 0x1p-9) + 0x1p-26);
+    const float target = (float)(u128_to_double(g) * 0x1p-80 * (1.0 + 0x1p-9) + 0x1p-18);
     uint32_t c[per], cs = 0;
     float m[per], ms = 0.0f;
 #pragma unroll
     for (int q = 0; q < per; ++q) {
         c[q] = S.pc[tid * per + q];
-        m[q] = use_mass ? S.pmf[tid * per + q] : 0.0f;
+        m[q] = use_mass ? (float)S.pm_lo[tid * per + q] * 0x1p-31f : 0.0f;
         cs += c[q];
         ms += m[q];
     }
@@ -1155,7 +1099,7 @@ FIE_DEV int binned_bound(FinSmem& S, int cnt, bool use_mass, u128 g)
     // every candidate's mass together is below g, beyond the float sums' error: the
     // crossing lies past the candidates
     const bool beyond = use_mass &&
-        (double)mall * (1.0 + 0x1p-9) + 0x1p-26 < u128_to_double(g) * 0x1p-80 * (1.0 - 0x1p-40);
+        (double)mall * (1.0 + 0x1p-9) + 0x1p-18 < u128_to_double(g) * 0x1p-80 * (1.0 - 0x1p-40);
     uint32_t crun = cb;
     float mrun = mb;
 #pragma unroll
@@ -1359,10 +1303,10 @@ FIE_DEV SortedScan sorted_scan(FinSmem& S, int nv, uint32_t tau)
             ++vcnt;
         }
     }
-    const u128 incl = wave_incl_scan_u128(sum);
+    const u128 incl = dwave_incl_scan_u128(sum);
     if (tau != 0) {                                   // uniform; tau == 0: every candidate survives
-        const u128 vw = wave_sum_u128(vsum);
-        const uint32_t vc = wave_sum_u32(vcnt);
+        const u128 vw = dwave_sum_u128(vsum);
+        const uint32_t vc = dwave_sum_u32(vcnt);
         if (lane == 63) {
             S.red128[kFinWaves + wave] = vw;
             S.red32[wave] = vc;
@@ -1417,7 +1361,7 @@ FIE_DEV void sorted_find(FinSmem& S, const SortedScan& sc, u128 g, int* slot_i, 
 // row: the full-row draw, and top-L logprobs deeper than the candidates.  Both
 // phases compute the same prologue (row maximum, tile table, row mass) from the
 // partials; a queued row's DeferRec carries what PH 1 cannot recompute cheaply.
-template <int DT, bool VEC, int PH, int Q>
+template <int DT, bool VEC, int PH, int Q, bool PRE>
 FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool inl, const bool hd = false)
 {
     const fie_sampler_args& a = P.a;
@@ -1462,20 +1406,23 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     if (bins || regs) {
         for (int i = tid; i < kPassBins; i += kFinThreads) {
             S.pc[i] = 0;
-            S.pmf[i] = 0.0f;
+            S.pm_lo[i] = 0;
         }
     }
+    // batches past the CU count are bound by traffic, and a row narrowed by mass may
+    // not need its candidates at all: there they are loaded after the row mass is known
+    const bool early = spec && (PRE || !bins);
     uint64_t xs[Q + 1];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         const int t = wave + kFinWaves * q;
-        xs[q] = spec && t < NT ? P.w.cand[((size_t)row * NT + t) * kCapW + lane] : 0ull;
+        xs[q] = early && t < NT ? P.w.cand[((size_t)row * NT + t) * kCapW + lane] : 0ull;
     }
     // Round 1: the row maximum, the safety bound and the candidate count, per wave.
     {
-        const uint64_t wm = wave_max_u64(pf_max);
-        const uint32_t wb = wave_max_u32(pf_bd);
-        const uint32_t wn = wave_sum_u32(pf_nc);
+        const uint64_t wm = dwave_max_u64(pf_max);
+        const uint32_t wb = dwave_max_u32(pf_bd);
+        const uint32_t wn = dwave_sum_u32(pf_nc);
         if (tid < NT) S.nc[tid] = pf_nc;
         if (lane == 0) {
             S.red64[wave] = wm;
@@ -1530,7 +1477,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
             if (need_mass) part = z ? (u128)tok_weight(y0, y0) * ct : (u128)ct * pf_sw;
         }
         if (need_mass) {
-            part = wave_sum_u128(part);
+            part = dwave_sum_u128(part);
             if (lane == 0) S.red128[wave] = part;
         }
     }
@@ -1544,32 +1491,48 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     // PH 0: the candidates as y-domain composites, those above the safety key into
     // S.cand (binned when narrowed by mass); tiles past the held ones load now.
     bool okr[Q + 1];             // the held slots, for the second sweep
-    if (spec) {
+    auto commit = [&]() {
         uint64_t best = 0;
-        {
-            const float rs = cand_rs(s);
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                const int t = wave + kFinWaves * q;
-                okr[q] = t < NT && (uint32_t)lane < S.nc[t];
-                xs[q] = okr[q] ? cand_y(xs[q], s, rs) : 0ull;
-            }
-            okr[Q] = tid == kFinThreads - 1;
-            xs[Q] = comp_key(k0, 0);
-            if (regs) cand_count(S, xs, okr, safe, best, bins, M);
+        if (early) {
+            if (regs) cand_count(S, xs, okr, safe, best, M);
             else cand_commit(S, xs, okr, safe, best, bins, M);
         }
         if (!regs)
-            for (int t0 = kFinWaves * Q; t0 < NT; t0 += kFinWaves * Q)
-                cand_batch<Q>(S, P, row, NT, t0, s, safe, best, bins, M, false, 0ull);
-        best = wave_max_u64(best);
+            for (int t0 = early ? kFinWaves * Q : 0; t0 < NT; t0 += kFinWaves * Q)
+                cand_batch<Q>(S, P, row, NT, t0, s, safe, best, bins, M, t0 == 0, comp_key(k0, 0));
+        best = dwave_max_u64(best);
         if (lane == 0 && best) atomicMax((unsigned long long*)&S.cmax, (unsigned long long)best);
+    };
+    if (spec) {
+        const float rs = cand_rs(s);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int t = wave + kFinWaves * q;
+            okr[q] = t < NT && (uint32_t)lane < S.nc[t];
+            xs[q] = okr[q] ? cand_y(xs[q], s, rs) : 0ull;
+        }
+        okr[Q] = tid == kFinThreads - 1;
+        xs[Q] = comp_key(k0, 0);
+        if (!bins) commit();
     }
     // Round 2: the row mass and the candidates.
     __syncthreads();
     u128 sall = 0;
     if (need_mass)
         for (int w = 0; w < kFinWaves; ++w) sall += S.red128[w];
+    // Rows narrowed by mass look for the mass past gmass (a top-p cut over the whole
+    // row, or a plain draw).  A weight is at most 2^80: when not even that many
+    // candidates could reach it, none of them is needed.
+    u128 gmass = 0;
+    bool far = false;
+    if (bins) {
+        if (sall != 0) gmass = tp < 1.0f ? ceil_mul_f32(tp, sall) - 1 : floor_mul_f64(urow, sall);
+        far = (u128)(ncall + 1) << 80 <= gmass;
+        if (!far) {
+            commit();
+            __syncthreads();
+        }
+    }
 
     int64_t token = -1;
     uint64_t tok_comp = 0;   // y-domain composite of the chosen token
@@ -1628,7 +1591,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         cmax = S.cmax;
 
 
-        if (nv > kSortMax) {
+        if (far || nv > kSortMax) {
             deep = true;
         } else {
             // what the selections below can reach: top-k and top-L by count; a
@@ -1642,8 +1605,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
             if (!greedy) {
                 if (mp > 0.0f) narrow = false;
                 else if (topk > 0) cnt = topk > cnt ? topk : cnt;
-                else if (tp < 1.0f) { by_mass = true; g = ceil_mul_f32(tp, sall) - 1; }
-                else { by_mass = true; g = floor_mul_f64(urow, sall); }
+                else { by_mass = true; g = gmass; }
                 if (by_mass && sall == 0) narrow = false;
             }
             nvall = nv;
@@ -1746,10 +1708,31 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         }
     }
 
-    // Full-row path for sampled rows the candidates could not settle.
+    // The LDS candidates again, for the logprobs of a row taken through a full-row path.
+    auto reload = [&]() {
+        sorted = false;
+        if (lp > 0 && n > 0) {
+            nv = load_candidates(S, P, row, NT, s, k0, safe);
+            if (nv <= kSortMax) {
+                sort_desc(S, nv);
+                sorted = true;
+            }
+        }
+    };
+
+    // Full-row path for sampled rows the candidates could not settle: at once, unless
+    // the row has span helpers or a threshold whose survivors are yet to be found.
     if (PH == 0 && !greedy && deep) {
-        defer(kDeferDraw);
-        return;
+        if (P.helpers || topk > 0 || mp > 0.0f ||
+            !windowed_deep<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, &cut, &T, &tok_comp)) {
+            defer(kDeferDraw);
+            return;
+        }
+        status |= FIE_ROW_EXACT_PATH;
+        tau = 0;
+        token = comp_idx(tok_comp);
+        if (a.tk_key && tid == 0) a.tk_key[row] = 0;
+        reload();
     }
     if (PH == 1 && !greedy && deep) {
         status |= FIE_ROW_EXACT_PATH;
@@ -1798,15 +1781,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         }
         token = comp_idx(tok_comp);
         if (a.tk_key && tid == 0) a.tk_key[row] = tk;
-        // the LDS candidates were overwritten: reload them for the logprobs below
-        sorted = false;
-        if (lp > 0 && n > 0) {
-            nv = load_candidates(S, P, row, NT, s, k0, safe);
-            if (nv <= kSortMax) {
-                sort_desc(S, nv);
-                sorted = true;
-            }
-        }
+        reload();
     }
 
     // Logprobs (sampler.py:262-291, rule R7): chosen token, then the row's best L,
@@ -1970,7 +1945,7 @@ FIE_DEV bool span_helper(FinSmem& S, const KParams& P, const int row, const int 
     if (pen)
         for (int i = tid; i < kSpan / 4; i += kFinThreads) ((uint4*)cnt)[i] = make_uint4(0, 0, 0, 0);
     {
-        const uint64_t wm = wave_max_u64(pf_max);
+        const uint64_t wm = dwave_max_u64(pf_max);
         if (lane == 0) S.red64[wave] = wm;
     }
     __syncthreads();
@@ -2038,8 +2013,8 @@ FIE_DEV bool span_helper(FinSmem& S, const KParams& P, const int row, const int 
             cv[k] = comp_key(fkey(y), (uint32_t)idx);
         }
     }
-    tail_n = wave_sum_u32(tail_n);
-    tail_w = wave_sum_u128(tail_w);
+    tail_n = dwave_sum_u32(tail_n);
+    tail_w = dwave_sum_u128(tail_w);
     if (lane == 0 && tail_n) {
         atomicAdd(&S.pc[kPassBins - 1], tail_n);
         bin_add(S, kPassBins - 1, tail_w);
@@ -2108,7 +2083,7 @@ __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KPar
             inl = false;
             hd = true;
         } else {
-            finish_row<DT, VEC, 0, 10>(S, P, blockIdx.x, true);
+            finish_row<DT, VEC, 0, 10, true>(S, P, blockIdx.x, true);
             __syncthreads();
             deep = S.dmode != 0;
             if (P.helpers && helped_row(P, blockIdx.x)) {
@@ -2118,9 +2093,9 @@ __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KPar
                 hd = true;
             }
         }
-        if (deep) finish_row<DT, VEC, 1, kReloadQ>(S, P, blockIdx.x, inl, hd);
+        if (deep) finish_row<DT, VEC, 1, kReloadQ, false>(S, P, blockIdx.x, inl, hd);
     } else {
-        finish_row<DT, VEC, 0, kReloadQ>(S, P, blockIdx.x, false);
+        finish_row<DT, VEC, 0, kReloadQ, false>(S, P, blockIdx.x, false);
     }
 }
 
@@ -2134,7 +2109,7 @@ __global__ __launch_bounds__(kFinThreads, 4) void k_deep(const KParams P)
     const uint32_t queued = P.w.dq[0];
     const uint32_t total = queued < (uint32_t)P.a.rows ? queued : (uint32_t)P.a.rows;
     if (blockIdx.x >= total) return;
-    finish_row<DT, VEC, 1, kReloadQ>(S, P, (int)P.w.dqrows[blockIdx.x], false);
+    finish_row<DT, VEC, 1, kReloadQ, false>(S, P, (int)P.w.dqrows[blockIdx.x], false);
 }
 
 }  // namespace fie

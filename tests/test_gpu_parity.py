@@ -642,3 +642,61 @@ def test_span_helpers_flat_rows_repeated(fs):
         out, _, _ = fs.step(xd, hp)
         assert (out["status"] & _lib.FIE_ROW_EXACT_PATH).sum() >= 4
         check(out, ref, params)
+
+
+def _deep_rows(rng, rows, vocab, dtype, kind):
+    """Rows whose cut or draw lies past the candidates: logits and a step (grid) they
+    are rounded to, so that thousands of tokens share a value."""
+    g = torch.Generator().manual_seed(int(rng.integers(1 << 30)))
+    x = torch.randn(rows, vocab, generator=g)
+    if kind == "flat":
+        x = 0.3 * x
+    elif kind == "peaked":
+        x = 0.5 * x - 1.1 * torch.log(torch.argsort(torch.rand(rows, vocab, generator=g), dim=1).float() + 1.0)
+    elif kind == "grid":                        # a few dozen values in all
+        x = torch.round(2.0 * x) / 2.0
+    elif kind == "wide":
+        x = 3.0 * x
+    elif kind == "constant":
+        x = torch.full_like(x, 1.25)
+    return x.to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind,vocab", [("flat", 40000), ("peaked", 151936), ("grid", 30001), ("wide", 65536),
+                                        ("constant", 12289)])
+def test_windowed_rows_match_the_oracle(fs, dtype, kind, vocab):
+    """Rows past the candidates in batches without span helpers: top-p and plain draws,
+    several temperatures, penalties (one history over 512 ids in one span), draws near
+    both ends."""
+    rng = np.random.default_rng(vocab)
+    rows = 20
+    x = _deep_rows(rng, rows, vocab, dtype, kind)
+    params, contexts = [], []
+    for i in range(rows):
+        pen = dict(presence_penalty=0.5, frequency_penalty=0.25, repetition_penalty=1.2) if i % 2 else {}
+        params.append(SamplingParams(temperature=(1.0, 0.7, 1.3)[i % 3], top_p=(0.95, 1.0, 0.99, 0.6)[i % 4],
+                                     logprobs=3 if i == 5 else None, **pen))
+        ids = rng.integers(0, vocab, 400)
+        if i == 3:
+            ids = np.concatenate([ids, np.full(700, 8200)])
+        contexts.append(ids.tolist())
+    uniforms = rng.random(rows)
+    uniforms[:4] = (0.0, 1.0 - 2.0 ** -53, 0.5, 0.999)
+    out, ref, _, _ = run_both(fs, x, params, uniforms, contexts, kept=False)
+    check(out, ref, params, lp=True)
+    assert int((out["status"] & _lib.FIE_ROW_EXACT_PATH != 0).sum()) > 0
+
+
+def test_windowed_rows_past_the_cu_count(fs):
+    """The same path in the 128-register kernel: 300 rows, each equal to itself in a
+    batch of 30."""
+    rng = np.random.default_rng(77)
+    x = _deep_rows(rng, 30, 20011, torch.bfloat16, "flat").to(DEV)
+    params = [SamplingParams(temperature=1.0, top_p=(0.9, 1.0)[i % 2]) for i in range(30)]
+    u = rng.random(30)
+    small, _, _ = fs.step(x, resolve_params(params, 20011, u, None))
+    small = {k: v.copy() for k, v in small.items()}
+    big, _, _ = fs.step(x.repeat(10, 1), resolve_params(params * 10, 20011, np.tile(u, 10), None))
+    for key in ("tokens", "cut_comp", "kept_mass", "status"):
+        np.testing.assert_array_equal(big[key], np.concatenate([small[key]] * 10), err_msg=key)
