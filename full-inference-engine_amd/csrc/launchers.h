@@ -18,8 +18,7 @@ hipError_t launch_finish_f32(const KParams& P, bool vec, bool deep, bool wide, h
 hipError_t launch_finish_f16(const KParams& P, bool vec, bool deep, bool wide, hipStream_t st);
 hipError_t launch_finish_bf16(const KParams& P, bool vec, bool deep, bool wide, hipStream_t st);
 
-// k_lmhead (fp16 / bf16 only).
-hipError_t launch_lmhead(const KParams& P, const void* hidden, const void* weight, int H, bool vec,
-                         bool longh, hipStream_t st);
+// The output layer: P.a.logits = hidden · weightᵀ (fp16 / bf16 only).
+hipError_t launch_lmhead(const KParams& P, const void* hidden, const void* weight, int H, hipStream_t st);
 
 }  // namespace fie

@@ -1,33 +1,21 @@
-// The lm_head projection with the sampler's streaming pass as its epilogue.
+// The lm_head projection in front of the sampler.
 //
 // The reference computes a decode step's logits with the model's output layer,
 // an nn.Linear without bias in the model dtype (continuous_batching.py:1345,1594,
 // 2225: `self._lm_head()(hidden)`), writes them to a buffer and hands that buffer
-// to the sampler (:1926-1928), whose first act is a full read of it.  k_lmhead
-// computes logits = hidden · weightᵀ on the matrix cores (bf16 or fp16 operands,
-// fp32 accumulation, rounded to nearest-even in the model dtype as the layer's
-// output is), writes them once for the passes that need the row again (the
-// full-row path, the kept-set check), and runs scan_tile over each 2048-token
-// tile it produced: the tile partials k_scan would have read back from HBM.
+// to the sampler (:1926-1928).  Here logits = hidden · weightᵀ is computed on the matrix
+// cores (bf16 or fp16 operands, fp32 accumulation over k in ascending steps of 32,
+// rounded to nearest-even in the model dtype as the layer's output is) and written
+// once; k_scan then reads it, mostly from the Infinity Cache.
+//
+// The weight is vocab x H and is read once whatever the batch, so small batches are
+// bound by HBM (1.25 GB at vocab 151936 and H 4096, 240 us at the rate of a large copy)
+// and large ones by the matrix cores and the LDS that feeds them.
 #pragma once
 
 #include "launchers.h"
 
 namespace fie {
-
-constexpr int kLhRows = 64;                   // rows per workgroup (4 groups of 16)
-constexpr int kLhThreads = 512;               // 8 waves: 4 row groups x 2 token groups
-constexpr int kLhWaves = kLhThreads / 64;
-constexpr int kLhSub = 128;                   // tokens per sub-block (64 per token group)
-constexpr int kLhK = 32;                      // K of one MFMA step
-constexpr int kLhKStage = 64;                 // K of one pipeline stage (two MFMA steps)
-constexpr int kLhStages = 3;                  // LDS stages (two in flight while one is used)
-constexpr int kLhRowsPerWave = kLhRows / kLhWaves;
-// One stage in 16-byte chunks: A 64 rows x 8, then B 128 tokens x 8; three per thread.
-constexpr int kLhChunksA = kLhRows * (kLhKStage / 8);
-constexpr int kLhChunks = kLhChunksA + kLhSub * (kLhKStage / 8);
-static_assert(kLhChunks == 3 * kLhThreads, "three chunks per thread per stage");
-static_assert(kLhKStage / kLhK == 2, "the fragment wait names two MFMA steps' operands");
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
@@ -64,225 +52,121 @@ FIE_DEV uint16_t round_logit(float v)
     }
 }
 
-// LDS: the GEMM's operand stages, then (reusing the space) the epilogue's
-// per-wave penalty counts and marks of one row's tile and the candidate staging
-// of scan_tile.
-template <bool LONGH>
-struct LhEpi {
-    uint32_t cnt[kLhWaves][LONGH ? kTile : kTile / 2];
-    uint32_t pbits[kLhWaves][kTile / 32];
-    uint64_t stage[kLhWaves][kStageW];
-    uint32_t uniq[kLhWaves];
-};
-template <bool LONGH>
-union LhSmem {
-    uint4 ops[kLhStages][kLhChunks];
-    LhEpi<LONGH> e;
-};
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-
-// s_waitcnt with vmcnt = n (n < 64) and no wait on the other counters.
-constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
-
-// 16 bytes of LDS at byte address `addr`, read by an instruction the compiler does
-// not track: its wait placement would otherwise drain every outstanding copy
-// into LDS before any LDS read.  The caller waits on lgkmcnt before use.
-FIE_DEV u32x4_t lds_read16(uint32_t addr)
+// Four consecutive tokens' logits of one row (the weight is the instruction's A, so a
+// lane's four results are neighbours in memory): one 8-byte store where `wide` (rows and
+// buffer 8-byte aligned) and all four are inside the vocabulary.
+template <int DT>
+FIE_DEV void store_logits(uint16_t* out, int64_t ld, int row, int tok, int V, bool wide, f32x4_t v)
 {
-    u32x4_t r;
-    asm volatile("ds_read_b128 %0, %1" : "=v"(r) : "v"(addr) : "memory");
-    return r;
+    uint16_t* p = out + (size_t)row * (size_t)ld + tok;
+    uint16_t h[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h[i] = round_logit<DT>(v[i]);
+    if (wide && tok + 4 <= V) {
+        *(uint2*)p = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (tok + i < V) p[i] = h[i];
+    }
 }
 
-FIE_DEV uint32_t lds_addr(const void* p)
-{
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
+// 64 WM rows by 64 WN tokens a workgroup of WM x WN waves, 64 x 64 each: 16 fragments
+// from LDS per 32 matrix instructions and 64 of k, the ratio at which the LDS reads
+// (128 bytes a cycle) take about as long as the instructions.  k goes in stages of 64
+// through two LDS buffers, one barrier a stage; the next two stages are in flight in
+// registers, and two workgroups share a CU where the buffers allow.
+//
+// Measured at vocab 151936, H 4096 (us; the GEMM fused with the scan that this replaces
+// took 677 at 16 rows and 1090 at 256, a library product takes 261 and 394):
+//   16 / 64 rows   1 x 4 waves 266 / 277, 1 x 2 waves 281 at 64; operands straight to
+//                  registers without LDS 264 / 430
+//   128 rows       2 x 2 waves 281, 2 x 4 waves 306
+//   256 rows       2 x 4 waves 382, 4 x 2 waves 408, 2 x 2 waves 421, 4 x 4 waves 676
+constexpr int kLhK = 64;
 
 // Chunk c (of 8) of operand row n sits at slot n * 8 + (c ^ (n & 7)): the eight
 // lanes one LDS cycle serves read eight rows' chunk c from eight distinct bank groups.
 FIE_DEV int lh_slot(int n, int c) { return n * 8 + (c ^ (n & 7)); }
 
-// Grid: 8 * ceil(NT / 8) * nrb workgroups.  Workgroups are dealt to the eight
-// XCDs round robin, so b, b + 8, b + 16, ... share one XCD; there, the nrb row
-// blocks of a tile come one after another and read the tile's weight rows
-// through that XCD's L2.
-template <int DT, bool VEC, bool LONGH>
-__global__ __launch_bounds__(kLhThreads, 4) void k_lmhead(const KParams P, const uint16_t* __restrict__ hid,
-                                                       const uint16_t* __restrict__ wt, int H, int nrb)
+// Grid: 8 * ceil(tiles / 8) * nrb workgroups.  Workgroups are dealt to the eight XCDs
+// round robin, so b, b + 8, b + 16, ... share one XCD; there, the nrb row blocks of a
+// tile come one after another and read its weight rows through that XCD's L2.
+template <int DT, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN, 2) void k_lmhead_tile(const uint16_t* __restrict__ hid,
+                                                               const uint16_t* __restrict__ wt, uint16_t* out,
+                                                               int64_t ld, int B, int V, int H, int nrb, int wide)
 {
-    constexpr int EPL = DTy<DT>::EPL, NL = kEPT / EPL;
-    __shared__ LhSmem<LONGH> L;
-    const fie_sampler_args& a = P.a;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int B = a.rows, V = a.vocab, NT = P.NT;
+    constexpr int BM = 64 * WM, BN = 64 * WN, TH = 64 * WM * WN;
+    constexpr int NC = (BM + BN) * (kLhK / 8) / TH;             // 16-byte chunks per thread and stage
+    __shared__ u32x4_t L[2][(BM + BN) * (kLhK / 8)];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
-    const int tile = 8 * (k / nrb) + xcd, rb = k % nrb;
-    if (tile >= NT) return;
-    if (blockIdx.x == 0 && tid < 2) P.w.dq[tid] = 0u;   // k_deep's queue, filled by k_finish
-    if (P.helpers && blockIdx.x == 0 && tid < B) P.w.harr[tid] = 0u;   // k_finish's arrivals
-    const int r0 = rb * kLhRows;
-    const int64_t ld = a.row_stride;
-    uint16_t* out = (uint16_t*)a.logits;
-
-    // 1. The GEMM, 128 tokens of the tile at a time (16 sub-blocks), K in stages of
-    //    64 through a three-stage LDS pipeline filled by direct global-to-LDS copies
-    //    (two stages in flight while one is read); one barrier per stage, no fence,
-    //    so the waits on the copies stay partial.  Wave (rg, tg) computes rows
-    //    r0 + 16 rg .. +15 by tokens 64 tg .. +63 of the sub-block.
-    const int rg = wv & 3, tg = wv >> 2;
-    const int nk = H / kLhKStage;
-    const int nsteps = (kTile / kLhSub) * nk;
-    // the copies this thread makes, one per 16-byte chunk: slots tid, tid + 512, tid + 1024
-    const uint16_t* src[3];
-    int sk[3];
+    const int t0 = (8 * (k / nrb) + xcd) * BN, r0 = (k % nrb) * BM;
+    if (t0 >= V) return;
+    const uint16_t* src[NC];
+    int dst[NC];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const int p = j * kLhThreads + tid;
-        const bool isa = p < kLhChunksA;
-        const int pp = isa ? p : p - kLhChunksA;
-        const int n = pp >> 3, c = (pp & 7) ^ (n & 7);
-        sk[j] = c * 8;
-        if (isa) {
-            const int row = r0 + n;
-            src[j] = hid + (size_t)(row < B ? row : 0) * H;
-        } else {
-            src[j] = nullptr;      // weight rows depend on the sub-block: set per copy
-            sk[j] |= n << 16;      // remember the token within the sub-block
-        }
+    for (int j = 0; j < NC; ++j) {
+        const int p = j * TH + tid, n = p >> 3, c = p & 7;
+        src[j] = (n < BM ? hid + (size_t)min(r0 + n, B - 1) * H : wt + (size_t)min(t0 + n - BM, V - 1) * H) + 8 * c;
+        dst[j] = lh_slot(n, c);
     }
-    auto issue = [&](int g) {
-        // the stage buffer follows g; past the end the source re-reads the start (unused)
-        lds_void_t* base = (lds_void_t*)&L.ops[g % kLhStages][0];
-        g = g < nsteps ? g : g - nsteps;
-        const int sb = g / nk, k0 = (g - sb * nk) * kLhKStage;
+    const int ns = H / kLhK;
+    u32x4_t ra[NC], rb[NC];
+    auto load = [&](u32x4_t (&r)[NC], int s) {
+        const int k0 = (s < ns ? s : ns - 1) * kLhK;            // past the end: again, unused
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const uint16_t* gp;
-            if (j == 0) {
-                gp = src[0] + k0 + sk[0];
-            } else {
-                const int tok = tile * kTile + sb * kLhSub + (sk[j] >> 16);
-                gp = wt + (size_t)(tok < V ? tok : 0) * H + k0 + (sk[j] & 0xFFFF);
-            }
-            __builtin_amdgcn_global_load_lds((const void*)gp,
-                                             (lds_void_t*)((__attribute__((address_space(3))) char*)base +
-                                                           (j * kLhThreads + wv * 64) * 16),
-                                             16, 0, 0);
+        for (int j = 0; j < NC; ++j) r[j] = *(const u32x4_t*)(src[j] + k0);
+    };
+    auto put = [&](const u32x4_t (&r)[NC], int b) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j) L[b][dst[j]] = r[j];
+    };
+    const int wr = wave % WM, wn = wave / WM;
+    f32x4_t acc[4][4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[m][q] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    auto mul = [&](int b) {
+#pragma unroll
+        for (int kk = 0; kk < kLhK / 32; ++kk) {
+            const int c = kk * 4 + (lane >> 4);
+            u32x4_t fh[4], fw[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) fh[m] = L[b][lh_slot(64 * wr + 16 * m + (lane & 15), c)];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) fw[q] = L[b][lh_slot(BM + 64 * wn + 16 * q + (lane & 15), c)];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[m][q] = mfma_16x16x32<DT>(fw[q], fh[m], acc[m][q]);
         }
     };
-    issue(0);
-    issue(1);
-    f32x4_t acc[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) acc[q] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    const int an = rg * 16 + (lane & 15);
-    for (int g = 0; g < nsteps; ++g) {
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(3));     // stage g has landed (g + 1 may not)
-        __builtin_amdgcn_s_barrier();
-        const uint32_t st = lds_addr(&L.ops[g % kLhStages][0]);
-        u32x4_t fa[kLhKStage / kLhK], fb[kLhKStage / kLhK][4];
-#pragma unroll
-        for (int kk = 0; kk < kLhKStage / kLhK; ++kk) {
-            const int c = kk * 4 + (lane >> 4);
-            fa[kk] = lds_read16(st + 16u * (uint32_t)lh_slot(an, c));
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                fb[kk][q] = lds_read16(st + 16u * (uint32_t)(kLhChunksA + lh_slot(tg * 64 + q * 16 + (lane & 15), c)));
-        }
-        // the wait names the fragments, so no use of them can be scheduled above it
-        asm volatile("s_waitcnt lgkmcnt(0)"
-                     : "+v"(fa[0]), "+v"(fa[1]), "+v"(fb[0][0]), "+v"(fb[0][1]), "+v"(fb[0][2]),
-                       "+v"(fb[0][3]), "+v"(fb[1][0]), "+v"(fb[1][1]), "+v"(fb[1][2]), "+v"(fb[1][3])
-                     :
-                     : "memory");
-#pragma unroll
-        for (int kk = 0; kk < kLhKStage / kLhK; ++kk) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc[q] = mfma_16x16x32<DT>(fa[kk], fb[kk][q], acc[q]);
-        }
-        // a finished sub-block's logits are stored before the next copies: stores
-        // count in vmcnt too, and issued first they cannot keep vmcnt(3) from
-        // meaning "the next stage has landed" (loads complete in issue order)
-        const int sb = g / nk;
-        if (g - sb * nk == nk - 1) {
-            const int n0 = tile * kTile + sb * kLhSub + tg * 64;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int tok = n0 + q * 16 + (lane & 15);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int row = r0 + rg * 16 + (lane >> 4) * 4 + i;
-                    if (row < B && tok < V) out[(size_t)row * ld + tok] = round_logit<DT>(acc[q][i]);
-                }
-                acc[q] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            }
-        }
-        issue(g + 2);
-    }
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));          // the copies past the end, before the space is reused
-    // every logit of the workgroup's tile is written before any wave reads it back
-    __threadfence();
+    load(ra, 0);
+    load(rb, 1);
+    put(ra, 0);
+    load(ra, 2);
     __syncthreads();
-
-    // 2. The epilogue: each wave takes 8 rows through scan_tile (k_scan's steps 3-6)
-    //    on the tile just written, which is still in this XCD's L2.  The penalty
-    //    counts come from k_prep's span bucket, as in k_scan, for this tile only.
-    const int lo = tile * kTile;
-    const int sp = tile / kWavesPerWG;
-    const uint32_t toff = (uint32_t)(lo - sp * kSpan);
-    uint32_t* cnt = L.e.cnt[wv];
-    uint32_t* pbits = L.e.pbits[wv];
-    for (int q = 0; q < kLhRowsPerWave; ++q) {
-        const int row = r0 + wv * kLhRowsPerWave + q;
-        if (row >= B) break;                                 // uniform in the wave
-        const RowCfg rc = row_cfg(a, row);
-        const size_t slot = (size_t)row * NT + tile;
-        const char* rowp = (const char*)a.logits + (size_t)row * (size_t)ld * 2;
-        uint4 raw[NL];
+    for (int s = 0; s < ns; s += 2) {           // H is a multiple of 128: ns is even
+        put(rb, 1);
+        load(rb, s + 3);
+        mul(0);
+        __syncthreads();
+        put(ra, 0);
+        load(ra, s + 4);
+        mul(1);
+        __syncthreads();
+    }
 #pragma unroll
-        for (int j = 0; j < NL; ++j) raw[j] = load_group<DT, VEC>(rowp, lo + (j * 64 + lane) * EPL, V);
-        if (rc.pen) {
-            for (int i = lane; i < (LONGH ? kTile : kTile / 2); i += 64) cnt[i] = 0;
-            for (int i = lane; i < kTile / 32; i += 64) pbits[i] = 0;
-            if (lane == 0) L.e.uniq[wv] = 0;
-            wave_lds_sync();
-            auto count = [&](uint32_t o) {
-                uint32_t was;
-                if (LONGH) {
-                    was = atomicAdd(&cnt[o], 1u);
-                } else {
-                    const uint32_t sh = (o & 1) * 16;
-                    was = (atomicAdd(&cnt[o >> 1], 1u << sh) >> sh) & 0xFFFFu;
-                }
-                if (was == 0) {
-                    atomicOr(&pbits[o >> 5], 1u << (o & 31));
-                    atomicAdd(&L.e.uniq[wv], 1u);
-                }
-            };
-            const size_t rs = (size_t)row * P.NS + sp;
-            const uint32_t nb = P.w.nb[rs];
-            if (nb <= (uint32_t)kBucketCap) {
-                for (uint32_t i = lane; i < nb; i += 64) {
-                    const uint32_t o = (uint32_t)P.w.bk[rs * kBucketCap + i] - toff;
-                    if (o < (uint32_t)kTile) count(o);
-                }
-            } else {
-                const int64_t h0 = a.hist_offsets[row], h1 = hist_end(a, row);
-                for (int64_t h = h0 + lane; h < h1; h += 64) {
-                    const uint32_t id = (uint32_t)a.hist_ids[h];
-                    const uint32_t o = id - (uint32_t)lo;
-                    if (id != 0 && id < (uint32_t)V && o < (uint32_t)kTile) count(o);
-                }
-            }
-            wave_lds_sync();
-            if (lane == 0) P.w.nu[slot] = L.e.uniq[wv];
-        } else if (lane == 0) {
-            P.w.nu[slot] = 0;
-        }
-        scan_tile<DT, LONGH>(P, rc, row, tile, raw, rowp, pbits, cnt, lo, L.e.stage[wv]);
-        wave_lds_sync();
+    for (int m = 0; m < 4; ++m) {
+        const int row = r0 + 64 * wr + 16 * m + (lane & 15);
+        if (row >= B) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            store_logits<DT>(out, ld, row, t0 + 64 * wn + 16 * q + 4 * (lane >> 4), V, wide, acc[m][q]);
     }
 }
 

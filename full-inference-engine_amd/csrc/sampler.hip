@@ -479,9 +479,9 @@ static int lmhead_run(const fie_sampler_args* args, const void* hidden, const vo
         rc = run_stage(P, FIE_STAGE_PREP, st);
         if (rc != FIE_OK) return rc;
     }
-    const bool vec = vec_ok(args->logits, args->row_stride, 2);
-    const bool longh = args->apply_penalties && args->max_row_hist > 65535;
-    rc = launch_status(launch_lmhead(P, hidden, weight, hidden_dim, vec, longh, st), "k_lmhead");
+    rc = launch_status(launch_lmhead(P, hidden, weight, hidden_dim, st), "k_lmhead");
+    if (rc != FIE_OK) return rc;
+    rc = run_stage(P, FIE_STAGE_SCAN, st);
     if (rc != FIE_OK || !whole) return rc;
     rc = run_stage(P, FIE_STAGE_FINISH, st);
     if (rc != FIE_OK || finish_in_place(P)) return rc;

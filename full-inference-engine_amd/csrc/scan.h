@@ -291,8 +291,7 @@ FIE_DEV RowCfg row_cfg(const fie_sampler_args& a, int row)
 // One wave's pass over one 2048-token tile of one row, its tokens already in
 // registers (raw, the lane layout of load_group): penalties, the tile maximum,
 // the tile mass and the candidates, written to the tile's partials.  `rowp` is
-// the row's token 0 for the re-read of penalised tokens (global memory, or a
-// producer's staging copy); pbits/cnt hold the penalty marks and counts of tokens
+// the row's token 0 for the re-read of penalised tokens; pbits/cnt hold the penalty marks and counts of tokens
 // pbase.. (u16 halves, u32 words when LONGH); `stage` is kStageW words of the
 // wave's own LDS.
 template <int DT, bool LONGH>

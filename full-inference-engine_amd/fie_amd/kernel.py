@@ -325,8 +325,8 @@ class FusedSampler:
     def launch_lmhead(self, args: SamplerArgs, hidden: torch.Tensor, weight: torch.Tensor,
                       kernel_only: bool = False) -> None:
         """The fused lm_head step: args.logits receives hidden @ weight.T and the
-        sampler runs on it (fie_sampler_lmhead_sample); with kernel_only, the fused
-        kernel alone (fie_sampler_lmhead_stage, for timing)."""
+        sampler runs on it (fie_sampler_lmhead_sample); with kernel_only, the projection
+        and the scan alone (fie_sampler_lmhead_stage, for timing)."""
         ws = self.ensure_workspace(args.rows, args.vocab)
         fn = self.lib.fie_sampler_lmhead_stage if kernel_only else self.lib.fie_sampler_lmhead_sample
         rc = fn(ctypes.byref(args), hidden.data_ptr(), weight.data_ptr(), hidden.shape[1], ctypes.byref(ws),

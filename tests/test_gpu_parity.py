@@ -700,3 +700,22 @@ def test_windowed_rows_past_the_cu_count(fs):
     big, _, _ = fs.step(x.repeat(10, 1), resolve_params(params * 10, 20011, np.tile(u, 10), None))
     for key in ("tokens", "cut_comp", "kept_mass", "status"):
         np.testing.assert_array_equal(big[key], np.concatenate([small[key]] * 10), err_msg=key)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,vocab,H", [(1, 63, 128), (16, 257, 384), (65, 777, 128), (128, 1030, 256),
+                                          (129, 515, 128), (300, 260, 384)])
+def test_lmhead_tile_edges(fs, dtype, rows, vocab, H):
+    """Row and token tiles left partly empty, rows whose stride is not a multiple of 8
+    bytes, one and several stages of k: every logit within one rounding of the fp32
+    product, or within the fp32 sums' error where it cancels."""
+    g = torch.Generator().manual_seed(rows + vocab)
+    hidden = torch.randn(rows, H, generator=g).to(dtype).to(DEV)
+    weight = torch.randn(vocab, H, generator=g).to(dtype).to(DEV)
+    hp = resolve_params([SamplingParams()] * rows, vocab, np.zeros(rows), None)
+    out, _, _, logits = fs.lmhead_step(hidden, weight, hp)
+    ref = hidden.float() @ weight.float().T
+    mag = hidden.float().abs() @ weight.float().abs().T
+    ulp = (logits.view(torch.int16).int() - ref.to(dtype).view(torch.int16).int()).abs()
+    assert bool(((ulp <= 1) | ((logits.float() - ref).abs() <= 32 * 2.0 ** -24 * mag)).all())
+    np.testing.assert_array_equal(out["tokens"], logits.float().argmax(1).cpu().numpy())
