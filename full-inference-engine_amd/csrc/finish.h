@@ -232,7 +232,7 @@ FIE_DEV SelResult lds_select(FinSmem& S, const uint64_t* cand, int n, const Pred
 // a dependent load; a span whose bucket overflowed is counted from the whole history.
 static_assert(kBucketCap == kFinThreads && kSpan == 2 * kChunk, "bucket entries per thread, chunks per span");
 
-template <int DT, bool VEC, class F>
+template <int DT, class F>
 FIE_DEV void row_pass(FinSmem& S, const KParams& P, int row, float s, bool pen, float rep,
                       float pres, float freq, uint32_t k0, F&& f)
 {
@@ -252,7 +252,7 @@ FIE_DEV void row_pass(FinSmem& S, const KParams& P, int row, float s, bool pen, 
     }
     auto issue = [&](int lo) {
 #pragma unroll
-        for (int j = 0; j < NL; ++j) nxt[j] = load_group<DT, VEC>(rowp, lo + (j * kFinThreads + tid) * EPL, V);
+        for (int j = 0; j < NL; ++j) nxt[j] = load_group<DT>(rowp, lo + (j * kFinThreads + tid) * EPL, V);
         if (pen) {
             // a chunk past the row's end reads the last span's entry, unused
             const int sp = lo / kSpan < P.NS ? lo / kSpan : P.NS - 1;
@@ -310,7 +310,7 @@ FIE_DEV void row_pass(FinSmem& S, const KParams& P, int row, float s, bool pen, 
 
 // Count (and mass) histogram of one digit level over the elements satisfying pr
 // whose composite bits above the digit equal `hiprefix`.
-template <int DT, bool VEC, bool MASS>
+template <int DT, bool MASS>
 FIE_DEV void pass_hist(FinSmem& S, const KParams& P, int row, float s, bool pen, float rep,
                        float pres, float freq, uint32_t k0, const Pred pr, int level,
                        uint64_t hiprefix)
@@ -323,7 +323,7 @@ FIE_DEV void pass_hist(FinSmem& S, const KParams& P, int row, float s, bool pen,
         if (MASS) { S.pm_lo[i] = 0; S.pm_hi[i] = 0; }
     }
     __syncthreads();
-    row_pass<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, [&](float y, uint32_t idx) {
+    row_pass<DT>(S, P, row, s, pen, rep, pres, freq, k0, [&](float y, uint32_t idx) {
         const uint64_t c = comp_key(fkey(y), idx);
         if ((top >= 64 || (c >> top) == hiprefix) && pr(c)) {
             const uint32_t d = (uint32_t)(c >> dg.shift) & dmask;
@@ -387,14 +387,14 @@ FIE_DEV int pass_pick(FinSmem& S, int nbins, u128 g)
 
 // Gather the elements satisfying pr whose composite bits from `top` up equal
 // `hiprefix` into S.cand; returns their number (the caller ensures <= kGCap).
-template <int DT, bool VEC>
+template <int DT>
 FIE_DEV int pass_gather(FinSmem& S, const KParams& P, int row, float s, bool pen, float rep,
                         float pres, float freq, uint32_t k0, const Pred pr, int top,
                         uint64_t hiprefix)
 {
     if (threadIdx.x == 0) S.n = 0;
     __syncthreads();
-    row_pass<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, [&](float y, uint32_t idx) {
+    row_pass<DT>(S, P, row, s, pen, rep, pres, freq, k0, [&](float y, uint32_t idx) {
         const uint64_t c = comp_key(fkey(y), idx);
         if ((top >= 64 || (c >> top) == hiprefix) && pr(c)) {
             const uint32_t at = atomicAdd(&S.n, 1u);
@@ -410,7 +410,7 @@ FIE_DEV int pass_gather(FinSmem& S, const KParams& P, int row, float s, bool pen
 // range fits in LDS, then the LDS selection.  When `have_l1` the level-0 pass
 // histogram for the same predicate is already in S (and `l1_adjust` has been
 // applied by the caller).
-template <int DT, bool VEC, bool MASS>
+template <int DT, bool MASS>
 FIE_DEV SelResult row_select(FinSmem& S, const KParams& P, int row, float s, bool pen, float rep,
                              float pres, float freq, uint32_t k0, const Pred pr, u128 g,
                              bool have_l1)
@@ -420,7 +420,7 @@ FIE_DEV SelResult row_select(FinSmem& S, const KParams& P, int row, float s, boo
     for (int level = 0; level < kLevels; ++level) {
         const Digit dg = kDigits[level];
         if (!(level == 0 && have_l1))
-            pass_hist<DT, VEC, MASS>(S, P, row, s, pen, rep, pres, freq, k0, pr, level, hiprefix);
+            pass_hist<DT, MASS>(S, P, row, s, pen, rep, pres, freq, k0, pr, level, hiprefix);
         const int b = pass_pick<MASS>(S, 1 << dg.bits, g);
         if (b < 0) return SelResult{0, excl + S.bex, 0, 0};
         const u128 above = S.bex;
@@ -430,7 +430,7 @@ FIE_DEV SelResult row_select(FinSmem& S, const KParams& P, int row, float s, boo
         excl += above;
         hiprefix = (hiprefix << dg.bits) | (uint64_t)b;
         if (cnt <= (uint32_t)kGCap) {
-            const int n = pass_gather<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, pr,
+            const int n = pass_gather<DT>(S, P, row, s, pen, rep, pres, freq, k0, pr,
                                                dg.shift, hiprefix);
             SelResult r = lds_select<MASS>(S, S.cand, n, pr, g);
             r.excl += excl;
@@ -549,7 +549,7 @@ FIE_DEV int dbin_pick(FinSmem& S, int bmax, u128 last, u128 g, u128* above)
 // and settled exactly among the elements of its one bin, gathered by a pass that
 // needs no weights.  Returns false (nothing decided) when a bin to be gathered
 // holds more than kGCap elements.
-template <int DT, bool VEC>
+template <int DT>
 FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pen, float rep,
                          float pres, float freq, uint32_t k0, float M, int topk, float mp, float tp,
                          double u, u128 sall, uint32_t* tk_out, uint32_t* tau_out, uint64_t* cut_out,
@@ -620,7 +620,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
             S.pm_hi[i] = 0;
         }
         __syncthreads();
-        row_pass<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, [&](float y, uint32_t idx) {
+        row_pass<DT>(S, P, row, s, pen, rep, pres, freq, k0, [&](float y, uint32_t idx) {
             const int b = dbin_y(M, y);
             atomicAdd(&S.pc[b], 1u);
             bin_add(S, b, weight_of(S, y, idx));
@@ -678,7 +678,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
         } else {
         if (tid == 0) S.n = 0;
         __syncthreads();
-        row_pass<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, [&](float y, uint32_t idx) {
+        row_pass<DT>(S, P, row, s, pen, rep, pres, freq, k0, [&](float y, uint32_t idx) {
             const int b = dbin_y(M, y);
             if ((b >= bl && b <= bh) || (b2l >= 0 && b >= b2l && b <= b2h)) {
                 const uint32_t at = atomicAdd(&S.n, 1u);
@@ -1361,7 +1361,7 @@ FIE_DEV void sorted_find(FinSmem& S, const SortedScan& sc, u128 g, int* slot_i, 
 // row: the full-row draw, and top-L logprobs deeper than the candidates.  Both
 // phases compute the same prologue (row maximum, tile table, row mass) from the
 // partials; a queued row's DeferRec carries what PH 1 cannot recompute cheaply.
-template <int DT, bool VEC, int PH, int Q, bool PRE>
+template <int DT, int PH, int Q, bool PRE>
 FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool inl, const bool hd = false)
 {
     const fie_sampler_args& a = P.a;
@@ -1724,7 +1724,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     // the row has span helpers or a threshold whose survivors are yet to be found.
     if (PH == 0 && !greedy && deep) {
         if (P.helpers || topk > 0 || mp > 0.0f ||
-            !windowed_deep<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, &cut, &T, &tok_comp)) {
+            !windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, &cut, &T, &tok_comp)) {
             defer(kDeferDraw);
             return;
         }
@@ -1738,21 +1738,21 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         status |= FIE_ROW_EXACT_PATH;
         cut = 0;
         uint32_t tk = 0;
-        const bool binned = binned_deep<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, M, topk, mp, tp,
+        const bool binned = binned_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, topk, mp, tp,
                                                  urow, sall, &tk, &tau, &cut, &T, &tok_comp, hd);
         if (!binned) {
         // radix levels over the composite, re-reading the row per level
         cut = 0;
         tk = 0;
         if (topk > 0) {
-            const SelResult r = row_select<DT, VEC, false>(S, P, row, s, pen, rep, pres, freq, k0,
+            const SelResult r = row_select<DT, false>(S, P, row, s, pen, rep, pres, freq, k0,
                                                            Pred{0, 0, 0}, (u128)(topk - 1), false);
             tk = comp_k(r.comp);
         }
         const uint32_t tmp = minp_key(M, mp);
         tau = tk > tmp ? tk : tmp;
         const Pred surv{tau, 0, 0};
-        pass_hist<DT, VEC, true>(S, P, row, s, pen, rep, pres, freq, k0, surv, 0, 0);
+        pass_hist<DT, true>(S, P, row, s, pen, rep, pres, freq, k0, surv, 0, 0);
         u128 part = 0;
         for (int b = tid; b < kPassBins; b += kFinThreads)
             part += ((u128)S.pm_hi[b] << 64) | S.pm_lo[b];
@@ -1760,7 +1760,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         bool l1 = true;
         if (tp < 1.0f) {
             const u128 thr = ceil_mul_f32(tp, Sv);
-            const SelResult r = row_select<DT, VEC, true>(S, P, row, s, pen, rep, pres, freq, k0,
+            const SelResult r = row_select<DT, true>(S, P, row, s, pen, rep, pres, freq, k0,
                                                           surv, thr - 1, true);
             cut = r.comp;
             T = r.excl + r.meas;
@@ -1769,12 +1769,12 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
             T = Sv;
         }
         if (T == 0) {
-            const SelResult r = row_select<DT, VEC, false>(S, P, row, s, pen, rep, pres, freq, k0,
+            const SelResult r = row_select<DT, false>(S, P, row, s, pen, rep, pres, freq, k0,
                                                            Pred{0, 0, 0}, 0, false);
             tok_comp = r.comp;
         } else {
             const u128 g = floor_mul_f64(urow, T);
-            const SelResult r = row_select<DT, VEC, true>(S, P, row, s, pen, rep, pres, freq, k0,
+            const SelResult r = row_select<DT, true>(S, P, row, s, pen, rep, pres, freq, k0,
                                                           Pred{tau, 0, cut}, g, l1);
             tok_comp = r.comp;
         }
@@ -1807,9 +1807,9 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
             } else {
                 // the L-th largest composite over the row, the L composites >= it
                 // gathered, then sorted by one thread
-                const SelResult r = row_select<DT, VEC, false>(S, P, row, s, pen, rep, pres, freq, k0,
+                const SelResult r = row_select<DT, false>(S, P, row, s, pen, rep, pres, freq, k0,
                                                                Pred{0, 0, 0}, (u128)(L - 1), false);
-                n = pass_gather<DT, VEC>(S, P, row, s, pen, rep, pres, freq, k0, Pred{0, 0, r.comp}, 64, 0);
+                n = pass_gather<DT>(S, P, row, s, pen, rep, pres, freq, k0, Pred{0, 0, r.comp}, 64, 0);
                 if (tid == 0) {
                     const int m = n < 32 ? n : 32;
                     uint64_t* top = S.cand;
@@ -1910,7 +1910,7 @@ FIE_DEV int arrive(FinSmem& S, const KParams& P, int row, uint32_t add, bool pub
 }
 
 // Returns true when this workgroup is to finish the row through the full-row path.
-template <int DT, bool VEC>
+template <int DT>
 FIE_DEV bool span_helper(FinSmem& S, const KParams& P, const int row, const int sp)
 {
     constexpr int EPL = DTy<DT>::EPL, SZ = DTy<DT>::SZ;
@@ -1928,7 +1928,7 @@ FIE_DEV bool span_helper(FinSmem& S, const KParams& P, const int row, const int 
     const char* rowp = (const char*)a.logits + (size_t)row * (size_t)a.row_stride * SZ;
     uint4 raw[NL];
 #pragma unroll
-    for (int j = 0; j < NL; ++j) raw[j] = load_group<DT, VEC>(rowp, lo + (j * kFinThreads + tid) * EPL, V);
+    for (int j = 0; j < NL; ++j) raw[j] = load_group<DT>(rowp, lo + (j * kFinThreads + tid) * EPL, V);
     const uint64_t pf_max = tid < NT ? P.w.maxc[(size_t)row * NT + tid] : 0ull;
     const size_t hs = (size_t)row * NS + sp;
     uint32_t nb = 0, of = 0;
@@ -2070,7 +2070,7 @@ FIE_DEV bool span_helper(FinSmem& S, const KParams& P, const int row, const int 
 // latency is the kernel's: with no more rows than CUs (one workgroup each) the WIDE
 // variant takes up to 256 registers a lane and spills nothing; larger batches take
 // 128 (two workgroups a CU).
-template <int DT, bool VEC, bool WIDE>
+template <int DT, bool WIDE>
 __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KParams P)
 {
     __shared__ FinSmem S;
@@ -2079,11 +2079,11 @@ __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KPar
         // with span helpers, in whichever of the row's workgroups arrives last
         bool deep, inl = true, hd = false;
         if (blockIdx.y > 0) {
-            deep = span_helper<DT, VEC>(S, P, blockIdx.x, blockIdx.y - 1);
+            deep = span_helper<DT>(S, P, blockIdx.x, blockIdx.y - 1);
             inl = false;
             hd = true;
         } else {
-            finish_row<DT, VEC, 0, 10, true>(S, P, blockIdx.x, true);
+            finish_row<DT, 0, 10, true>(S, P, blockIdx.x, true);
             __syncthreads();
             deep = S.dmode != 0;
             if (P.helpers && helped_row(P, blockIdx.x)) {
@@ -2093,23 +2093,23 @@ __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KPar
                 hd = true;
             }
         }
-        if (deep) finish_row<DT, VEC, 1, kReloadQ, false>(S, P, blockIdx.x, inl, hd);
+        if (deep) finish_row<DT, 1, kReloadQ, false>(S, P, blockIdx.x, inl, hd);
     } else {
-        finish_row<DT, VEC, 0, kReloadQ, false>(S, P, blockIdx.x, false);
+        finish_row<DT, 0, kReloadQ, false>(S, P, blockIdx.x, false);
     }
 }
 
 // A fixed grid taking queued rows one at a time; every workgroup leaves once the
 // queue is drained (the count is final: k_finish has completed).  The queue is
 // short in decode (a few rows a step) but holds every row of a flat batch.
-template <int DT, bool VEC>
+template <int DT>
 __global__ __launch_bounds__(kFinThreads, 4) void k_deep(const KParams P)
 {
     __shared__ FinSmem S;
     const uint32_t queued = P.w.dq[0];
     const uint32_t total = queued < (uint32_t)P.a.rows ? queued : (uint32_t)P.a.rows;
     if (blockIdx.x >= total) return;
-    finish_row<DT, VEC, 1, kReloadQ, false>(S, P, (int)P.w.dqrows[blockIdx.x], false);
+    finish_row<DT, 1, kReloadQ, false>(S, P, (int)P.w.dqrows[blockIdx.x], false);
 }
 
 }  // namespace fie

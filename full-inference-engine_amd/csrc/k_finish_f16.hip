@@ -4,19 +4,12 @@
 
 namespace fie {
 
-hipError_t launch_finish_f16(const KParams& P, bool vec, bool deep, bool wide, hipStream_t st)
+hipError_t launch_finish_f16(const KParams& P, bool deep, bool wide, hipStream_t st)
 {
-    if (deep) {
-        // one workgroup per queue slot; those past the queued count leave at once
-        if (vec) k_deep<FIE_F16, true><<<P.a.rows, kFinThreads, 0, st>>>(P);
-        else k_deep<FIE_F16, false><<<P.a.rows, kFinThreads, 0, st>>>(P);
-    } else if (vec) {
-        if (wide) k_finish<FIE_F16, true, true><<<dim3(P.a.rows, P.helpers ? P.NS + 1 : 1), kFinThreads, 0, st>>>(P);
-        else k_finish<FIE_F16, true, false><<<P.a.rows, kFinThreads, 0, st>>>(P);
-    } else {
-        if (wide) k_finish<FIE_F16, false, true><<<dim3(P.a.rows, P.helpers ? P.NS + 1 : 1), kFinThreads, 0, st>>>(P);
-        else k_finish<FIE_F16, false, false><<<P.a.rows, kFinThreads, 0, st>>>(P);
-    }
+    // k_deep: one workgroup per queue slot; those past the queued count leave at once
+    if (deep) k_deep<FIE_F16><<<P.a.rows, kFinThreads, 0, st>>>(P);
+    else if (wide) k_finish<FIE_F16, true><<<dim3(P.a.rows, P.helpers ? P.NS + 1 : 1), kFinThreads, 0, st>>>(P);
+    else k_finish<FIE_F16, false><<<P.a.rows, kFinThreads, 0, st>>>(P);
     return hipGetLastError();
 }
 

@@ -75,7 +75,7 @@ __global__ __launch_bounds__(kPrepThreads) void k_prep(const KParams P)
 constexpr int kArgChunk = 8192;   // tokens per workgroup of the argmax pass
 
 // Chunk maxima of the raw logits (token 0 included, no penalties, no scaling).
-template <int DT, bool VEC>
+template <int DT>
 __global__ __launch_bounds__(kScanThreads) void k_argmax_scan(const void* logits, int V,
                                                               int64_t stride, int NT,
                                                               uint64_t* maxc)
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(kScanThreads) void k_argmax_scan(const void* logits
     const char* rowp = (const char*)logits + (size_t)row * (size_t)stride * SZ;
     uint4 raw[NL];
 #pragma unroll
-    for (int j = 0; j < NL; ++j) raw[j] = load_group<DT, VEC>(rowp, lo + (j * kScanThreads + tid) * EPL, V);
+    for (int j = 0; j < NL; ++j) raw[j] = load_group<DT>(rowp, lo + (j * kScanThreads + tid) * EPL, V);
     uint32_t tm = 0, ti = 0xFFFFFFFFu;
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(64) void k_argmax_finish(const uint64_t* maxc, int 
 }
 
 // ---------------------------------------------------------------- kept set
-template <int DT, bool VEC>
+template <int DT>
 __global__ __launch_bounds__(kScanThreads) void k_kept(const KParams P, uint8_t* kept, float* probs)
 {
     constexpr int EPL = DTy<DT>::EPL, SZ = DTy<DT>::SZ, NL = kArgChunk / kScanThreads / EPL;
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(kScanThreads) void k_kept(const KParams P, uint8_t*
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
         const int e0 = lo + (j * kScanThreads + tid) * EPL;
-        const uint4 raw = load_group<DT, VEC>(rowp, e0, V);
+        const uint4 raw = load_group<DT>(rowp, e0, V);
 #pragma unroll
         for (int e = 0; e < EPL; ++e) {
             const int idx = e0 + e;
@@ -318,11 +318,6 @@ static int check_args(const fie_sampler_args* a)
     return FIE_OK;
 }
 
-static bool vec_ok(const void* p, int64_t stride, int sz)
-{
-    return ((uintptr_t)p % 16) == 0 && ((stride * sz) % 16) == 0;
-}
-
 #define FIE_LAUNCH_CHECK(what)                                                          \
     do {                                                                                \
         hipError_t e_ = hipGetLastError();                                              \
@@ -360,8 +355,6 @@ static bool finish_in_place(const KParams& P) { return P.a.rows <= cu_count(); }
 
 static int run_stage(const KParams& P, int stage, hipStream_t st)
 {
-    const int sz = P.a.dtype == FIE_F32 ? 4 : 2;
-    const bool vec = vec_ok(P.a.logits, P.a.row_stride, sz);
     const bool longh = P.a.apply_penalties && P.a.max_row_hist > 65535;
     if (stage == FIE_STAGE_PREP) {
         if (P.a.apply_penalties) {
@@ -373,15 +366,15 @@ static int run_stage(const KParams& P, int stage, hipStream_t st)
     hipError_t e;
     const char* what;
     if (stage == FIE_STAGE_SCAN) {
-        e = launch_scan(P, vec, longh, st);
+        e = launch_scan(P, longh, st);
         what = "k_scan";
     } else {
         const bool deep = stage == FIE_STAGE_DEEP;
         const bool wide = finish_in_place(P);
         switch (P.a.dtype) {
-        case FIE_F32: e = launch_finish_f32(P, vec, deep, wide, st); break;
-        case FIE_F16: e = launch_finish_f16(P, vec, deep, wide, st); break;
-        default: e = launch_finish_bf16(P, vec, deep, wide, st); break;
+        case FIE_F32: e = launch_finish_f32(P, deep, wide, st); break;
+        case FIE_F16: e = launch_finish_f16(P, deep, wide, st); break;
+        default: e = launch_finish_bf16(P, deep, wide, st); break;
         }
         what = deep ? "k_deep" : "k_finish";
     }
@@ -523,19 +516,13 @@ int fie_sampler_argmax(const void* logits, int32_t dtype, int32_t rows, int32_t 
     int rc = ws_of(ws, rows, vocab, &w);
     if (rc != FIE_OK) return rc;
     const int NT = (vocab + kArgChunk - 1) / kArgChunk;
-    const int sz = dtype == FIE_F32 ? 4 : 2;
-    const bool vec = vec_ok(logits, row_stride, sz);
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid(NT, rows);
-#define FIE_ARGMAX(DT)                                                                                   \
-    if (vec) k_argmax_scan<DT, true><<<grid, kScanThreads, 0, st>>>(logits, vocab, row_stride, NT, w.maxc); \
-    else k_argmax_scan<DT, false><<<grid, kScanThreads, 0, st>>>(logits, vocab, row_stride, NT, w.maxc);
     switch (dtype) {
-    case FIE_F32: FIE_ARGMAX(FIE_F32) break;
-    case FIE_F16: FIE_ARGMAX(FIE_F16) break;
-    default: FIE_ARGMAX(FIE_BF16) break;
+    case FIE_F32: k_argmax_scan<FIE_F32><<<grid, kScanThreads, 0, st>>>(logits, vocab, row_stride, NT, w.maxc); break;
+    case FIE_F16: k_argmax_scan<FIE_F16><<<grid, kScanThreads, 0, st>>>(logits, vocab, row_stride, NT, w.maxc); break;
+    default: k_argmax_scan<FIE_BF16><<<grid, kScanThreads, 0, st>>>(logits, vocab, row_stride, NT, w.maxc); break;
     }
-#undef FIE_ARGMAX
     FIE_LAUNCH_CHECK("k_argmax_scan");
     k_argmax_finish<<<(rows + 63) / 64, 64, 0, st>>>(w.maxc, NT, rows, tokens);
     FIE_LAUNCH_CHECK("k_argmax_finish");
@@ -548,19 +535,13 @@ int fie_sampler_kept(const fie_sampler_args* args, uint8_t* kept, float* probs,
     KParams P;
     int rc = prepare(args, ws, &P);
     if (rc != FIE_OK || args->rows == 0) return rc;
-    const int sz = args->dtype == FIE_F32 ? 4 : 2;
-    const bool vec = vec_ok(args->logits, args->row_stride, sz);
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid((args->vocab + kArgChunk - 1) / kArgChunk, args->rows);
-#define FIE_KEPT(DT)                                                                  \
-    if (vec) k_kept<DT, true><<<grid, kScanThreads, 0, st>>>(P, kept, probs);        \
-    else k_kept<DT, false><<<grid, kScanThreads, 0, st>>>(P, kept, probs);
     switch (args->dtype) {
-    case FIE_F32: FIE_KEPT(FIE_F32) break;
-    case FIE_F16: FIE_KEPT(FIE_F16) break;
-    default: FIE_KEPT(FIE_BF16) break;
+    case FIE_F32: k_kept<FIE_F32><<<grid, kScanThreads, 0, st>>>(P, kept, probs); break;
+    case FIE_F16: k_kept<FIE_F16><<<grid, kScanThreads, 0, st>>>(P, kept, probs); break;
+    default: k_kept<FIE_BF16><<<grid, kScanThreads, 0, st>>>(P, kept, probs); break;
     }
-#undef FIE_KEPT
     FIE_LAUNCH_CHECK("k_kept");
     return FIE_OK;
 }

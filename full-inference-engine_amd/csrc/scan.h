@@ -124,12 +124,27 @@ FIE_DEV float lane_get(const uint4& r, int e)
     }
 }
 
+// 16 bytes at an address aligned to the element only: rows of an odd vocabulary start
+// anywhere, and the target's unaligned access mode loads them with the one instruction
+// aligned rows take (element by element they took 8 loads and cost k_scan 35%, the
+// full-row passes 60%).
+template <int SZ> struct Raw16;
+template <> struct Raw16<2> { typedef uint32_t T __attribute__((ext_vector_type(4), aligned(2))); };
+template <> struct Raw16<4> { typedef uint32_t T __attribute__((ext_vector_type(4), aligned(4))); };
+
+template <int DT>
+FIE_DEV uint4 load16(const char* p)
+{
+    const typename Raw16<DTy<DT>::SZ>::T v = *(const typename Raw16<DTy<DT>::SZ>::T*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 // One 16-byte group of tokens [e0, e0 + EPL) of a row; tokens at or past V read 0.
-template <int DT, bool VEC>
+template <int DT>
 FIE_DEV uint4 load_group(const char* rowp, int e0, int V)
 {
     constexpr int EPL = DTy<DT>::EPL, SZ = DTy<DT>::SZ;
-    if (VEC && e0 + EPL <= V) return *(const uint4*)(rowp + (size_t)e0 * SZ);
+    if (e0 + EPL <= V) return load16<DT>(rowp + (size_t)e0 * SZ);
     uint4 r = make_uint4(0, 0, 0, 0);
     uint32_t* w = &r.x;
 #pragma unroll
@@ -576,7 +591,7 @@ FIE_DEV void scan_tile(const KParams& P, const RowCfg& rc, int row, int tile,
 }
 
 // ---------------------------------------------------------------- k_scan
-template <int DT, bool VEC, bool LONGH>
+template <int DT, bool LONGH>
 __global__ __launch_bounds__(kScanThreads) void k_scan(const KParams P)
 {
     constexpr int EPL = DTy<DT>::EPL, SZ = DTy<DT>::SZ, NL = kEPT / EPL;
@@ -610,7 +625,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(const KParams P)
     uint4 raw[NL];
 #pragma unroll
     for (int j = 0; j < NL; ++j)
-        raw[j] = live ? load_group<DT, VEC>(rowp, lo + (j * 64 + lane) * EPL, V) : make_uint4(0, 0, 0, 0);
+        raw[j] = live ? load_group<DT>(rowp, lo + (j * 64 + lane) * EPL, V) : make_uint4(0, 0, 0, 0);
 
     // 2. Penalty counts of the span's ids (sampler.py:134-144), shared by the four
     //    waves.  A token's first count sets its bit in pbits and counts it as a

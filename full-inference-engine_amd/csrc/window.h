@@ -301,7 +301,7 @@ FIE_DEV bool tile_markstein(const float (&x)[kEPT])
 // overflowed.  The next tile's loads are in flight while one is processed.
 enum { kWinCount, kWinSub, kWinWeigh };
 
-template <int DT, bool VEC>
+template <int DT>
 FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s, bool pen, float rep, float pres,
                       float freq, float M, float y0, bool has_cut, u128& m0, u128& m1)
 {
@@ -372,12 +372,12 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
         // are then the same at every step
         const int tt = t < NT ? t : NT - 1;
         const int lo = tt * kTile;
-        if (VEC && lo + kTile <= V) {
+        if (lo + kTile <= V) {
 #pragma unroll
-            for (int j = 0; j < NL; ++j) nxt[j] = *(const uint4*)(rowp + (size_t)(lo + (j * 64 + lane) * EPL) * SZ);
+            for (int j = 0; j < NL; ++j) nxt[j] = load16<DT>(rowp + (size_t)(lo + (j * 64 + lane) * EPL) * SZ);
         } else {
 #pragma unroll
-            for (int j = 0; j < NL; ++j) nxt[j] = load_group<DT, VEC>(rowp, lo + (j * 64 + lane) * EPL, V);
+            for (int j = 0; j < NL; ++j) nxt[j] = load_group<DT>(rowp, lo + (j * 64 + lane) * EPL, V);
         }
         if (pen) {
             const size_t sr = (size_t)row * P.NS + tt / kWavesPerWG;
@@ -566,7 +566,7 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
 
 // The row's cut and draw (top_p tp, uniform u, whole-row mass sall) over its whole
 // vocabulary.  Returns false when it decided nothing.
-template <int DT, bool VEC>
+template <int DT>
 FIE_DEV bool windowed_deep(FinSmem& S, const KParams& P, int row, float s, bool pen, float rep, float pres,
                            float freq, uint32_t k0, float M, float tp, double u, u128 sall, uint64_t* cut_out,
                            u128* T_out, uint64_t* tok_out)
@@ -585,7 +585,7 @@ FIE_DEV bool windowed_deep(FinSmem& S, const KParams& P, int row, float s, bool 
         if (tid == 0) S.wn = 0;
         __syncthreads();
         u128 m0 = 0, m1 = 0;
-        win_pass<DT, VEC>(S, P, row, phase, s, pen, rep, pres, freq, M, y0, has_cut, m0, m1);
+        win_pass<DT>(S, P, row, phase, s, pen, rep, pres, freq, M, y0, has_cut, m0, m1);
         bool lost = false;
         if (phase == kWinWeigh) {
             // the exact selections (rules R3, R4) inside the windows
