@@ -1740,7 +1740,10 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         uint32_t tk = 0;
         const bool binned = binned_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, topk, mp, tp,
                                                  urow, sall, &tk, &tau, &cut, &T, &tok_comp, hd);
-        if (!binned) {
+        // a bin too full to gather (16-bit logits share values): by windows, or
+        if (!binned && !(topk == 0 && !(mp > 0.0f) &&
+                         windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, &cut, &T,
+                                           &tok_comp))) {
         // radix levels over the composite, re-reading the row per level
         cut = 0;
         tk = 0;

@@ -719,3 +719,16 @@ def test_lmhead_tile_edges(fs, dtype, rows, vocab, H):
     ulp = (logits.view(torch.int16).int() - ref.to(dtype).view(torch.int16).int()).abs()
     assert bool(((ulp <= 1) | ((logits.float() - ref).abs() <= 32 * 2.0 ** -24 * mag)).all())
     np.testing.assert_array_equal(out["tokens"], logits.float().argmax(1).cpu().numpy())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_helper_rows_with_shared_values(fs, dtype):
+    """Rows with span helpers (at most 16 a batch) on logits of a few dozen values: the
+    helpers' bins hold more tokens than can be gathered."""
+    rng = np.random.default_rng(11)
+    x = _deep_rows(rng, 12, 60001, dtype, "grid")
+    params = [SamplingParams(temperature=(1.0, 0.8)[i % 2], top_p=(0.95, 1.0, 0.99)[i % 3],
+                             presence_penalty=0.3 * (i % 2)) for i in range(12)]
+    contexts = [rng.integers(0, 60001, 200).tolist() for _ in range(12)]
+    out, ref, _, _ = run_both(fs, x, params, rng.random(12), contexts, kept=False)
+    check(out, ref, params)
