@@ -103,6 +103,60 @@ FIE_DEV float weight40(float d)
     return __builtin_floorf(__builtin_ldexpf(p, (int)n + 40));
 }
 
+// cexp(d) * 2^20 before any floor, for d <= 0 or NaN: weight40(d) = floor(weight20(d) *
+// 2^20), bit for bit.  The quotient's integer part comes from adding 1.5 * 2^23 + 20
+// (nearest even, as rint, since the constant is even), whose low bits then hold n + 20
+// for the exponent: two adds and a shifted add where rint, a conversion, an add and a
+// ldexp took twice the cycles (the f32 adds issue at twice the rate of those).
+FIE_DEV float weight20(float d)
+{
+    constexpr float kMagic = 12582932.0f;
+    const float dc = d > -80.0f ? d : -80.0f;
+    const float t = dc * 1.44269502f + kMagic;
+    const float n = t - kMagic;
+    float r = __builtin_fmaf(n, -0.693145752f, dc);
+    r = __builtin_fmaf(n, -1.42860677e-06f, r);
+    float p = 1.98412701e-04f;
+    p = __builtin_fmaf(p, r, 1.38888892e-03f);
+    p = __builtin_fmaf(p, r, 8.33333377e-03f);
+    p = __builtin_fmaf(p, r, 4.16666679e-02f);
+    p = __builtin_fmaf(p, r, 1.66666672e-01f);
+    p = __builtin_fmaf(p, r, 0.5f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    return __uint_as_float((__float_as_uint(t) << 23) + __float_as_uint(p));
+}
+
+// The exact integer sum of the weights of one lane's tokens, eight at a time.  With
+// v = weight20(d), a weight is floor(v) * 2^20 + floor(fract(v) * 2^20), both parts at
+// most 2^20.  Added, rounding down, to a float in [2^23, 2^24), whose unit is 1, each
+// part floors itself, and eight of them stay within the range: three instructions a
+// token, where a floor, a conversion to fp64 and an fp64 add took 1.5 times the cycles.
+// The rounding mode is changed and restored inside the one asm statement.
+struct WeightSum {
+    uint32_t hi = 0, lo = 0;     // sums of the float accumulators' bits, their bias removed
+
+    FIE_DEV void add8(const float (&v)[8])
+    {
+        float h = 0x1p23f, l = 0x1p23f, t;
+        asm("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n"
+            "v_fract_f32 %2, %3\n v_add_f32 %0, %0, %3\n v_fma_f32 %1, %2, %11, %1\n"
+            "v_fract_f32 %2, %4\n v_add_f32 %0, %0, %4\n v_fma_f32 %1, %2, %11, %1\n"
+            "v_fract_f32 %2, %5\n v_add_f32 %0, %0, %5\n v_fma_f32 %1, %2, %11, %1\n"
+            "v_fract_f32 %2, %6\n v_add_f32 %0, %0, %6\n v_fma_f32 %1, %2, %11, %1\n"
+            "v_fract_f32 %2, %7\n v_add_f32 %0, %0, %7\n v_fma_f32 %1, %2, %11, %1\n"
+            "v_fract_f32 %2, %8\n v_add_f32 %0, %0, %8\n v_fma_f32 %1, %2, %11, %1\n"
+            "v_fract_f32 %2, %9\n v_add_f32 %0, %0, %9\n v_fma_f32 %1, %2, %11, %1\n"
+            "v_fract_f32 %2, %10\n v_add_f32 %0, %0, %10\n v_fma_f32 %1, %2, %11, %1\n"
+            "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
+            : "+&v"(h), "+&v"(l), "=&v"(t)
+            : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]), "s"(0x1p20f));
+        hi += __float_as_uint(h) - 0x4B000000u;
+        lo += __float_as_uint(l) - 0x4B000000u;
+    }
+    FIE_DEV uint64_t total() const { return ((uint64_t)hi << 20) + lo; }
+};
+
 // x / s correctly rounded by Markstein's correction from r = RN(1/s):
 // q = RN(x r), e = x - q s (exact by FMA), RN(q + e r).  Exact (equal to the IEEE
 // quotient) when the quotient and the intermediates stay normal; callers keep
@@ -322,6 +376,13 @@ FIE_DEV uint32_t dpp_mov(uint32_t v)
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
 
 FIE_DEV uint32_t rl(uint32_t v, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, lane); }
+
+// A value that is the same in every lane, into scalar registers.
+FIE_DEV uint64_t uni64(uint64_t v)
+{
+    return ((uint64_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+           (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+}
 
 FIE_DEV uint32_t dwave_max_u32(uint32_t v)
 {

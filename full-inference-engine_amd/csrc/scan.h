@@ -264,6 +264,20 @@ FIE_DEV uint32_t ballot_select(const uint32_t (&k)[N], uint32_t target, uint32_t
     return pre;
 }
 
+// Whether every token of the tile (NaN aside) is inside Markstein's range (finite fp16
+// values always are, and 0 gives 0).
+template <int DT>
+FIE_DEV bool tile_markstein(const float (&x)[kEPT])
+{
+    float hi = 0.0f, lo = __builtin_inff();
+#pragma unroll
+    for (int i = 0; i < kEPT; ++i) {
+        hi = __builtin_fmaxf(hi, __builtin_fabsf(x[i]));
+        if (DT != FIE_F16) lo = __builtin_fminf(lo, __builtin_fabsf(x[i]));
+    }
+    return __ballot(hi > 0x1p96f || lo < 0x1p-96f) == 0;
+}
+
 // LDS of k_scan.
 template <bool LONGH>
 struct ScanSmem {
@@ -341,6 +355,7 @@ FIE_DEV void scan_tile(const KParams& P, const RowCfg& rc, int row, int tile,
 #pragma unroll
     for (int q = 0; q < kPS; ++q) { pv[q] = __builtin_nanf(""); pidx[q] = 0xFFFFFFFFu; }
     bool odd = false;        // a patched value outside the unchecked divide's range
+    bool patched = false;    // some of the wave's x[] are penalised in place
     if (pen) {
         uint32_t mine = 0;   // bit i: the lane's token i is penalised
 #pragma unroll
@@ -352,6 +367,7 @@ FIE_DEV void scan_tile(const KParams& P, const RowCfg& rc, int row, int tile,
             return LONGH ? cnt[o] : ((cnt[o >> 1] >> ((o & 1) * 16)) & 0xFFFFu);
         };
         if (__ballot(__builtin_popcount(mine) > kPS) != 0) {
+            patched = true;
             for (uint32_t b = mine; b; b &= b - 1) {
                 const int i = __builtin_ctz(b);
                 const int o = lo - pbase + ((i / EPL) * 64 + lane) * EPL + (i % EPL);
@@ -433,47 +449,46 @@ FIE_DEV void scan_tile(const KParams& P, const RowCfg& rc, int row, int tile,
     const uint32_t fi = dwave_min_u32(first);
     if (lane == 0) P.w.maxc[slot] = km ? comp_key(km, fi) : 0ull;
 
-    // 5. Tile mass relative to the tile maximum (rule R1): the integer weights
-    //    floor(cexp(y - m_t) 2^40) < 2^41 as integer-valued floats, summed in fp64,
-    //    which is exact (a lane's 32 weights stay below 2^46).  y - m_t needs no
-    //    folding of -0: both zeros give the same difference.  The temperature
+    // 5. Tile mass relative to the tile maximum (rule R1): the exact integer sum of the
+    //    weights floor(cexp(y - m_t) 2^40).  y - m_t needs no folding of -0: both
+    //    zeros give the same difference.  The temperature
     //    divide is Markstein's corrected product, equal to the IEEE quotient while
     //    2^-96 <= |x| <= 2^96 and 2^-30 <= s <= 2^30: always so for finite,
     //    nonzero fp16 logits; 0 gives 0; +-inf and NaN give NaN there and weight 0
     //    through cexp's clamp, as the IEEE quotient's weight does.  Only penalised
     //    values can leave the range, and the patch step flags them.
     if (need_mass) {
-        double acc = 0.0;
+        uint64_t acc = 0;
         if (km != 0) {
             const float mt = y_of_xkey(km, s);
-            if (s == 1.0f) {
+            WeightSum ws;
+            auto sum = [&](auto yof) {
 #pragma unroll
-                for (int i = 0; i < kEPT; ++i) acc += (double)weight40(x[i] - mt);
+                for (int i = 0; i < kEPT; i += 8) {
+                    float v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = weight20(yof(x[i + k]) - mt);
+                    ws.add8(v);
+                }
+            };
+            if (s == 1.0f) {
+                sum([&](float v) { return v; });
             } else if (s >= 0x1p-30f && s <= 0x1p30f) {
                 const float rs = 1.0f / s;
-                if (DT == FIE_F16 && __ballot(odd) == 0) {
-#pragma unroll
-                    for (int i = 0; i < kEPT; ++i) acc += (double)weight40(div_markstein(x[i], s, rs) - mt);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < kEPT; ++i) {
-                        const float y = markstein_ok(x[i]) ? div_markstein(x[i], s, rs) : x[i] / s;
-                        acc += (double)weight40(y - mt);
-                    }
-                }
+                if (DT == FIE_F16 ? __ballot(odd) == 0 : tile_markstein<DT>(x))
+                    sum([&](float v) { return div_markstein(v, s, rs); });
+                else
+                    sum([&](float v) { return markstein_ok(v) ? div_markstein(v, s, rs) : v / s; });
             } else {
-#pragma unroll
-                for (int i = 0; i < kEPT; ++i) acc += (double)weight40(scaled(x[i], s) - mt);
+                sum([&](float v) { return scaled(v, s); });
             }
-        }
-        if (km != 0) {
-            const float mt = y_of_xkey(km, s);
+            acc = ws.total();
 #pragma unroll
             for (int q = 0; q < kPS; ++q)
                 if (__ballot(pidx[q] != 0xFFFFFFFFu) != 0)
-                    acc += (double)weight40((s == 1.0f ? pv[q] : scaled(pv[q], s)) - mt);
+                    acc += (uint64_t)weight40((s == 1.0f ? pv[q] : scaled(pv[q], s)) - mt);
         }
-        const uint64_t tot = dwave_sum_u64((uint64_t)acc);
+        const uint64_t tot = dwave_sum_u64(acc);
         if (lane == 0) P.w.sw[slot] = tot;
     }
 
@@ -525,11 +540,38 @@ FIE_DEV void scan_tile(const KParams& P, const RowCfg& rc, int row, int tile,
         uint32_t E;
         uint32_t at = dwave_excl_scan_u32((uint32_t)(__builtin_popcount(mask) + __builtin_popcount(pmask)), &E);
         uint64_t* st = stage;
-        for (uint32_t b = mask; b; b &= b - 1) {
-            const int i = __builtin_ctz(b);
-            if (at < (uint32_t)kStageW)
-                st[at] = comp_key(fkey(pick32(x, (uint32_t)i) + 0.0f), (uint32_t)elem_index<EPL>(lo, lane, i));
+        auto put = [&](float v, uint32_t idx) {
+            if (at < (uint32_t)kStageW) st[at] = comp_key(fkey(v + 0.0f), idx);
             ++at;
+        };
+        if (patched) {
+            for (uint32_t b = mask; b; b &= b - 1) {
+                const int i = __builtin_ctz(b);
+                put(pick32(x, (uint32_t)i), (uint32_t)elem_index<EPL>(lo, lane, i));
+            }
+        } else {
+            // the values from memory again (the lines were just read), a lane's first
+            // kHeld tokens in one round trip: taking them from the registers by a
+            // runtime index is 31 selects a token (k_scan 2-4 us slower on 256 rows)
+            constexpr int kHeld = 4;
+            uint32_t b = mask, hi[kHeld];
+            float hv[kHeld];
+#pragma unroll
+            for (int q = 0; q < kHeld; ++q) {
+                if (b) {
+                    hi[q] = (uint32_t)elem_index<EPL>(lo, lane, __builtin_ctz(b));
+                    hv[q] = load_elem<DT>(rowp, hi[q]);
+                }
+                b &= b - 1;
+            }
+            const int have = __builtin_popcount(mask);
+#pragma unroll
+            for (int q = 0; q < kHeld; ++q)
+                if (q < have) put(hv[q], hi[q]);
+            for (b = have > kHeld ? b : 0u; b; b &= b - 1) {
+                const uint32_t idx = (uint32_t)elem_index<EPL>(lo, lane, __builtin_ctz(b));
+                put(load_elem<DT>(rowp, idx), idx);
+            }
         }
         if (__ballot(pmask != 0) != 0) {
 #pragma unroll

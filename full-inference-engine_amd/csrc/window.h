@@ -279,18 +279,6 @@ FIE_DEV float win_y(float x, float s, float rs)
     return scaled(x, s);
 }
 
-// Whether every token of the tile (NaN aside) is inside Markstein's range.
-FIE_DEV bool tile_markstein(const float (&x)[kEPT])
-{
-    float hi = 0.0f, lo = __builtin_inff();
-#pragma unroll
-    for (int i = 0; i < kEPT; ++i) {
-        hi = __builtin_fmaxf(hi, __builtin_fabsf(x[i]));
-        lo = __builtin_fminf(lo, __builtin_fabsf(x[i]));
-    }
-    return __ballot(hi > 0x1p96f || lo < 0x1p-96f) == 0;
-}
-
 // One pass over the row, a wave per tile: tokens counted per bin (kWinCount), those of
 // the windows in `big` per finer bin (kWinSub), or weighed (kWinWeigh): the exact mass
 // above each window into m0, m1, the windows' tokens into S.cand.
@@ -448,7 +436,7 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
         } else {
             // the scaled logits in place of the logits
             if (s != 1.0f) {
-                if (DT == FIE_F16 || tile_markstein(x)) {
+                if (DT == FIE_F16 || tile_markstein<DT>(x)) {
 #pragma unroll
                     for (int i = 0; i < kEPT; ++i) x[i] = div_markstein(x[i], s, rs);
                 } else {
