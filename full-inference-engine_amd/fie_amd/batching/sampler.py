@@ -77,11 +77,11 @@ class ParamTable:
     """Per-row columns of a batch's SamplingParams, from one pass over the objects.
 
     A decode loop passes the same SamplingParams objects step after step (each
-    request keeps its own); the last table is reused when the batch holds exactly the
-    same objects in the same order.  The table keeps those objects alive, so an
+    request keeps its own); a sampler reuses its last table when the batch holds exactly
+    the same objects in the same order.  The table keeps those objects alive, so an
     identity match cannot be a new object at a recycled address."""
 
-    __slots__ = ("objs", "greedy", "pen", "temps", "top_k", "top_p", "min_p", "lp",
+    __slots__ = ("wants_logprobs", "plain", "any_pen", "shared", "own", "objs", "greedy", "pen", "temps", "top_k", "top_p", "min_p", "lp",
                  "rep", "pres", "freq", "seeded", "seeds", "_resolved")
 
     def __init__(self, params: list[SamplingParams]):
@@ -104,6 +104,12 @@ class ParamTable:
         self.seeded = np.array(cols[10], dtype=bool)
         self.seeds = np.array(cols[11], dtype=np.uint64) if rows else np.zeros(0, np.uint64)
         self._resolved: dict[int, tuple] = {}
+        # what sample() asks of the whole batch
+        self.wants_logprobs = bool((self.lp >= 0).any())
+        self.plain = bool((self.greedy & ~self.pen).all())
+        self.any_pen = bool(self.pen.any())
+        self.shared = np.nonzero(~self.greedy & ~self.seeded)[0]      # rows of the shared stream
+        self.own = np.nonzero(~self.greedy & self.seeded)[0].tolist()  # rows of their own
 
     def resolved(self, vocab: int) -> tuple:
         """(scale, top_k, top_p, min_p, flags) as the kernels take them, resolved the way
@@ -124,32 +130,23 @@ class ParamTable:
         return len(params) == len(objs) and all(map(operator.is_, params, objs))
 
 
-_last_table: list[ParamTable | None] = [None]
-
-
-def param_table(params: list[SamplingParams]) -> ParamTable:
-    t = _last_table[0]
-    if t is None or not t.matches(params):
-        t = ParamTable(params)
-        _last_table[0] = t
-    return t
-
-
 def resolve_params(params: list[SamplingParams], vocab: int, uniforms: np.ndarray | None,
                    contexts: list[list[int]] | None, rng: np.ndarray | None = None,
                    history: DeviceHistory | None = None,
-                   request_ids: list[object] | None = None) -> HostParams:
+                   request_ids: list[object] | None = None,
+                   table: ParamTable | None = None) -> HostParams:
     """Per-row arrays for the kernels, derived the way sampler.py:109,182-192 does.
     The draws are `uniforms` (float64 [rows]) or, when `rng` (uint64 [rows, 3]) is
     given, derived on the device from it.  With a `history` and `request_ids` the
     penalty contexts are kept on the device across steps (only appended tokens
-    move); otherwise they are packed afresh."""
+    move); otherwise they are packed afresh.  `table` is the batch's ParamTable when the
+    caller has it."""
     rows = len(params)
     if uniforms is None:
         uniforms = np.zeros(rows, dtype=np.float64)
-    t = param_table(params)
-    greedy, pen, temps, top_k, top_p, min_p = t.greedy, t.pen, t.temps, t.top_k, t.top_p, t.min_p
-    apply = bool(pen.any()) and contexts is not None
+    t = table if table is not None else ParamTable(params)
+    pen = t.pen
+    apply = t.any_pen and contexts is not None
     ends = dst = src = None
     if apply and history is not None and request_ids is not None:
         offsets, ends, invalid, longest, dst, src = history.update(contexts, pen, request_ids, vocab)
@@ -226,22 +223,32 @@ class BatchedSampler:
             self._seeded.pop(request_id, None)
         self._history.forget(request_ids)
 
+    # the last step's parameters: a decode loop passes the same objects again
+    _table: ParamTable | None = None
+
+    def _params(self, params: list[SamplingParams]) -> ParamTable:
+        t = self._table
+        if t is None or not t.matches(params):
+            t = self._table = ParamTable(params)
+        return t
+
     def _draw_keys(self, params: list[SamplingParams],
                    request_ids: list[object] | None) -> np.ndarray:
         """uint64 [rows, 3] (key0, key1, counter) per row: a seeded row's request
         stream at its next position, the shared stream in row order otherwise
         (greedy rows draw nothing)."""
-        rows = len(params)
-        t = param_table(params)
-        keys = np.zeros((rows, 3), dtype=np.uint64)
-        shared = np.nonzero(~t.greedy & ~t.seeded)[0]
+        return self._keys_of(self._params(params), request_ids)
+
+    def _keys_of(self, t: ParamTable, request_ids: list[object] | None) -> np.ndarray:
+        keys = np.zeros((len(t.objs), 3), dtype=np.uint64)
+        shared = t.shared
         if shared.size:
             keys[shared, 0] = self._shared_key
             keys[shared, 1] = SHARED_STREAM
             keys[shared, 2] = np.arange(self._shared_draws + 1, self._shared_draws + 1 + shared.size,
                                         dtype=np.uint64)
             self._shared_draws += int(shared.size)
-        for r in np.nonzero(~t.greedy & t.seeded)[0].tolist():
+        for r in t.own:
             rid = request_ids[r] if request_ids is not None else r
             keys[r] = (int(t.seeds[r]), SEEDED_STREAM, self._next_draw(rid))
         return keys
@@ -269,19 +276,17 @@ class BatchedSampler:
 
         # the per-row predicates from one pass over the params (reused while a decode
         # loop passes the same SamplingParams objects)
-        t = param_table(params)
-        wants_logprobs = bool((t.lp >= 0).any())
-        plain = bool((t.greedy & ~t.pen).all())
-        if plain and not wants_logprobs:
+        t = self._params(params)
+        if t.plain and not t.wants_logprobs:
             # sampler.py:103-106: one argmax kernel and one device-to-host copy.
             return SampleResult(self._fused.argmax(logits).tolist(), {})
 
         hp = resolve_params(params, vocab, None, context_tokens,
-                            rng=self._draw_keys(params, request_ids),
-                            history=self._history, request_ids=request_ids)
+                            rng=self._keys_of(t, request_ids),
+                            history=self._history, request_ids=request_ids, table=t)
         out, _, _ = self._fused.step(logits, hp)
         tokens = out["tokens"].tolist()
-        return SampleResult(tokens, self._logprobs(params, tokens, out) if wants_logprobs else {})
+        return SampleResult(tokens, self._logprobs(params, tokens, out) if t.wants_logprobs else {})
 
     @staticmethod
     def _logprobs(params: list[SamplingParams], chosen: list[int],

@@ -125,7 +125,18 @@ class DeviceStep:
         self.host_np = self.host.numpy()
         self.base = self.dev.data_ptr()
         self.param_bytes = self.out_begin
+        # views of the pinned block, made once: (name, view) of the parameters, the
+        # history's starts and ends, the outputs
+        self._params = [(name, name in _TABLE_FIELDS, self.host_view(name, dt, rows * width))
+                        for name, dt, width in PARAM_FIELDS]
+        self._hist_off = self.host_view("hist_off", np.int64, rows + 1)
+        self._hist_end = self.host_view("hist_end", np.int64, rows)
+        self._outputs = {name: self.host_view(name, dt, rows * w).reshape(rows, w) if w > 1
+                         else self.host_view(name, dt, rows) for name, dt, w in OUTPUT_FIELDS}
+        self._out_dev, self._out_host = self.dev[self.out_begin:], self.host[self.out_begin:]
+        self._up = (0, None, None)        # the last upload's size and views
         self._staged: dict[str, np.ndarray] = {}
+        self._args: SamplerArgs | None = None   # the block's own pointers (args_of)
 
     def host_view(self, name: str, dtype, count: int) -> np.ndarray:
         o = self.offs[name]
@@ -139,19 +150,19 @@ class DeviceStep:
         # the parameter table of an unchanged batch, which nothing writes) is already
         # in place; draws and the history fields are copied every step
         last = self._staged
-        for name, dt, width in PARAM_FIELDS:
+        for name, table, view in self._params:
             src = getattr(hp, name)
             if src is None:
                 continue
-            if name in _TABLE_FIELDS:
+            if table:
                 if last.get(name) is src:
                     continue
                 last[name] = src
-            self.host_view(name, dt, self.rows * width)[:] = np.asarray(src).reshape(-1)
-        self.host_view("hist_off", np.int64, len(hp.hist_off))[:] = hp.hist_off
+            view[:] = np.asarray(src).reshape(-1)
+        self._hist_off[:len(hp.hist_off)] = hp.hist_off
         if hp.hist_ends is not None:
             # device-resident history: row ranges, then the appended (position, id) pairs
-            self.host_view("hist_end", np.int64, self.rows)[:] = hp.hist_ends
+            self._hist_end[:] = hp.hist_ends
             n = int(hp.hist_write_dst.shape[0])
             o = self.offs["hist_ids"]
             self.host_np[o:o + 8 * n].view(np.int64)[:] = hp.hist_write_dst
@@ -164,24 +175,47 @@ class DeviceStep:
         # history ids are the tail of the parameter block: upload only what is used
         self.param_bytes = self.offs["hist_ids"] + 4 * n
 
+    def _copy_up(self) -> None:
+        n = self.param_bytes
+        if self._up[0] != n:
+            self._up = (n, self.dev[:n], self.host[:n])
+        self._up[1].copy_(self._up[2], non_blocking=True)
+
     def upload(self, stream: torch.cuda.Stream) -> None:
         if stream == torch.cuda.current_stream(self.dev.device):
-            self.dev[:self.param_bytes].copy_(self.host[:self.param_bytes], non_blocking=True)
+            self._copy_up()
             return
         with torch.cuda.stream(stream):
-            self.dev[:self.param_bytes].copy_(self.host[:self.param_bytes], non_blocking=True)
+            self._copy_up()
 
     def download(self, stream: torch.cuda.Stream) -> None:
         if stream == torch.cuda.current_stream(self.dev.device):
-            self.host[self.out_begin:].copy_(self.dev[self.out_begin:], non_blocking=True)
+            self._out_host.copy_(self._out_dev, non_blocking=True)
             return
         with torch.cuda.stream(stream):
-            self.host[self.out_begin:].copy_(self.dev[self.out_begin:], non_blocking=True)
+            self._out_host.copy_(self._out_dev, non_blocking=True)
 
     def outputs(self) -> dict[str, np.ndarray]:
-        return {name: self.host_view(name, dt, self.rows * w).reshape(self.rows, w)
-                if w > 1 else self.host_view(name, dt, self.rows)
-                for name, dt, w in OUTPUT_FIELDS}
+        return dict(self._outputs)
+
+    def args_of(self) -> SamplerArgs:
+        """A new argument struct holding the block's own pointers."""
+        a = SamplerArgs()
+        if self._args is None:
+            b = SamplerArgs()
+            b.lp_cols = LP_COLS
+            b.scale, b.top_k, b.top_p, b.min_p = map(self.ptr, ("scale", "top_k", "top_p", "min_p"))
+            b.flags, b.logprobs, b.uniform = map(self.ptr, ("flags", "logprobs", "uniform"))
+            b.repetition, b.presence, b.frequency = map(self.ptr, ("rep", "pres", "freq"))
+            b.hist_offsets, b.hist_ids = self.ptr("hist_off"), self.ptr("hist_ids")
+            b.tokens, b.status, b.tk_key = map(self.ptr, ("tokens", "status", "tk_key"))
+            b.cut_comp, b.row_max = self.ptr("cut_comp"), self.ptr("row_max")
+            b.kept_mass, b.row_mass = self.ptr("kept_mass"), self.ptr("row_mass")
+            b.chosen_logprob = self.ptr("chosen_lp")
+            b.top_ids, b.top_logprobs = self.ptr("top_ids"), self.ptr("top_lp")
+            self._args = b
+        ctypes.memmove(ctypes.byref(a), ctypes.byref(self._args), ctypes.sizeof(a))
+        return a
 
 
 class FusedSampler:
@@ -244,30 +278,22 @@ class FusedSampler:
     def build_args(self, logits: torch.Tensor, buf: DeviceStep, hp: HostParams) -> SamplerArgs:
         logits, dt = self._logits_info(logits)
         rows, vocab = logits.shape
-        a = SamplerArgs()
+        a = buf.args_of()
         a.logits = logits.data_ptr()
         a.dtype = dt
         a.rows = rows
         a.vocab = vocab
-        a.lp_cols = LP_COLS
         a.row_stride = logits.stride(0)
-        a.scale, a.top_k, a.top_p, a.min_p = (buf.ptr("scale"), buf.ptr("top_k"),
-                                              buf.ptr("top_p"), buf.ptr("min_p"))
-        a.flags, a.logprobs, a.uniform = buf.ptr("flags"), buf.ptr("logprobs"), buf.ptr("uniform")
-        a.apply_penalties = 1 if hp.apply_penalties else 0
+        if hp.apply_penalties:
+            a.apply_penalties = 1
         a.max_row_hist = int(hp.max_row_hist)
-        a.repetition, a.presence, a.frequency = buf.ptr("rep"), buf.ptr("pres"), buf.ptr("freq")
-        a.hist_offsets, a.hist_ids = buf.ptr("hist_off"), buf.ptr("hist_ids")
         if hp.hist_ends is not None:
             a.hist_ends = buf.ptr("hist_end")
             a.hist_ids = hp.hist_store.ids.data_ptr()
-        a.hist_invalid = buf.ptr("hist_invalid") if hp.hist_invalid is not None else None
-        a.tokens, a.status, a.tk_key = buf.ptr("tokens"), buf.ptr("status"), buf.ptr("tk_key")
-        a.cut_comp, a.row_max = buf.ptr("cut_comp"), buf.ptr("row_max")
-        a.kept_mass, a.row_mass = buf.ptr("kept_mass"), buf.ptr("row_mass")
-        a.chosen_logprob = buf.ptr("chosen_lp")
-        a.top_ids, a.top_logprobs = buf.ptr("top_ids"), buf.ptr("top_lp")
-        a.rng = buf.ptr("rng") if hp.rng is not None else None
+        if hp.hist_invalid is not None:
+            a.hist_invalid = buf.ptr("hist_invalid")
+        if hp.rng is not None:
+            a.rng = buf.ptr("rng")
         a._keep = logits  # the converted tensor must outlive the launch
         return a
 
@@ -381,12 +407,12 @@ class FusedSampler:
         lib = self.lib
         n = int(hp.hist_write_dst.shape[0]) if hp.hist_ends is not None else 0
         ids_ptr = hp.hist_store.ids.data_ptr() if n else 0
-        buf.upload(stream)
+        buf._copy_up()
         if n:
             o = buf.ptr("hist_ids")
             _lib.check(lib.fie_sampler_history_write(ids_ptr, o, o + 8 * n, n, sptr),
                        "fie_sampler_history_write")
         _lib.check(lib.fie_sampler_sample(ctypes.byref(args), ctypes.byref(ws), sptr), "fie_sampler_sample")
-        buf.download(stream)
+        buf._out_host.copy_(buf._out_dev, non_blocking=True)
         stream.synchronize()
         return buf.outputs(), args, buf

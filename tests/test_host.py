@@ -471,3 +471,19 @@ def test_argmax_and_cexp_argument_errors():
     assert lib.fie_sampler_argmax(None, 0, 1, 10, 10, None, None, None) == _lib.FIE_E_ARG
     assert lib.fie_sampler_cexp(None, None, -1, None) == _lib.FIE_E_ARG
     assert lib.fie_sampler_cexp(None, None, 0, None) == _lib.FIE_OK
+
+
+def test_each_sampler_keeps_its_own_parameter_table():
+    """Samplers used in turn reuse their own last table; a batch with other objects, in
+    another order or of another length gets a new one, with its own columns."""
+    a, b = _NoKernels(generator_seed=1), _NoKernels(generator_seed=2)
+    p = [SamplingParams(temperature=1.0, top_k=5), SamplingParams(temperature=0.5, logprobs=2)]
+    q = [SamplingParams(), SamplingParams()]
+    ta, tb = a._params(p), b._params(q)
+    assert a._params(list(p)) is ta and b._params(q) is tb
+    assert ta.wants_logprobs and not ta.plain and tb.plain and not tb.wants_logprobs
+    turned = a._params(p[::-1])
+    assert turned is not ta and turned.top_k.tolist() == [0, 5]
+    assert a._params(p[:1]).top_k.tolist() == [5]
+    own = resolve_params(q, 100, None, None, table=tb)
+    assert own.flags.tolist() == resolve_params(q, 100, None, None).flags.tolist()
