@@ -1720,11 +1720,15 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         }
     };
 
+    // The windowed path's list may run on into the row's candidate slots unless the
+    // logprobs read the candidates again.
+    const WinList list{P.w.cand + (size_t)row * NT * kCapW, (uint32_t)(kGCap + (lp > 0 ? 0 : NT * kCapW))};
+
     // Full-row path for sampled rows the candidates could not settle: at once, unless
     // the row has span helpers or a threshold whose survivors are yet to be found.
     if (PH == 0 && !greedy && deep) {
         if (P.helpers || topk > 0 || mp > 0.0f ||
-            !windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, &cut, &T, &tok_comp)) {
+            !windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, list, &cut, &T, &tok_comp)) {
             defer(kDeferDraw);
             return;
         }
@@ -1742,8 +1746,8 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
                                                  urow, sall, &tk, &tau, &cut, &T, &tok_comp, hd);
         // a bin too full to gather (16-bit logits share values): by windows, or
         if (!binned && !(topk == 0 && !(mp > 0.0f) &&
-                         windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, &cut, &T,
-                                           &tok_comp))) {
+                         windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, list, &cut,
+                                           &T, &tok_comp))) {
         // radix levels over the composite, re-reading the row per level
         cut = 0;
         tk = 0;

@@ -32,7 +32,7 @@ constexpr int kWinBins = kWinOctaves * (1 << kWinOct) + 1;
 // powers of two (and of those over common temperatures) that 16-bit logits lie on.
 constexpr float kWinOne = 1.000337f;
 constexpr int kSubBits = 12, kSubBins = 1 << kSubBits;   // bins of a refining count
-constexpr int kWinCap = kGCap;             // tokens gathered, both windows together
+constexpr int kWinSplit = kGCap / 2;       // a window with more tokens is narrowed to one bin
 constexpr int kIdxBits = 19;               // token indexes are below 2^19
 constexpr uint32_t kIdxMask = (1u << kIdxBits) - 1;
 static_assert(kMaxTiles * kTile <= 1 << kIdxBits, "index bits of a packed composite");
@@ -78,7 +78,7 @@ FIE_DEV float win_mass(const FinSmem& S, const Win& w, int k, int j, float M)
 // hold too many tokens, to the one bin that f lies in: two neighbouring values shared
 // by thousands each could not be told apart by a finer count of both.  False when the
 // mass does not get there.
-FIE_DEV bool win_pick(FinSmem& S, int k, bool sub, float M, float f, float eps)
+FIE_DEV bool win_pick(FinSmem& S, int k, bool sub, bool pen, float M, float f, float eps)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nb = sub ? kSubBins : kWinBins, per = (nb + kFinThreads - 1) / kFinThreads;
@@ -148,7 +148,7 @@ FIE_DEV bool win_pick(FinSmem& S, int k, bool sub, float M, float f, float eps)
         }
         __syncthreads();
         above = S.wab;
-        const bool wide = found && eps > 0.0f && S.wch - S.wcl > (uint32_t)kWinCap / 2;
+        const bool wide = found && eps > 0.0f && S.wch - S.wcl > (uint32_t)kWinSplit;
         if (!wide) break;
         eps = 0.0f;
         __syncthreads();
@@ -168,7 +168,9 @@ FIE_DEV bool win_pick(FinSmem& S, int k, bool sub, float M, float f, float eps)
             const float yh = l <= 1 ? M : (M - edge(l)) + 0.0f, yl = (M - edge(h + 1)) + 0.0f;
             v.hi = ((uint64_t)fkey(yh) << kIdxBits) | kIdxMask;
             v.lo = (uint64_t)fkey(yl) << kIdxBits;
-            v.byidx = 1;          // should it be refined: 16-bit logits mostly put one value in a bin
+            // should it be refined: 16-bit logits mostly put one value in a bin, but for
+            // a few penalised tokens among them
+            v.byidx = pen ? 0 : 1;
         }
         v.n = S.wch - S.wcl;
         v.above = above;
@@ -183,17 +185,31 @@ FIE_DEV bool win_pick(FinSmem& S, int k, bool sub, float M, float f, float eps)
     return found;
 }
 
-// The gathered composites S.cand[0, n) inside the packed range [lo, hi], in rank order:
+// The gathered list: its first kGCap composites in LDS, the rest (16-bit logits: a value
+// shared by over 4096 tokens of a 152k vocabulary, which two more counts of the row would
+// narrow in 130 us) in the row's candidate slots of the workspace, when those are free.
+struct WinList {
+    uint64_t* more;
+    uint32_t cap;
+    FIE_DEV uint64_t get(const FinSmem& S, int i) const { return i < kGCap ? S.cand[i] : more[i - kGCap]; }
+    FIE_DEV void put(FinSmem& S, uint32_t at, uint64_t c) const
+    {
+        if (at < (uint32_t)kGCap) S.cand[at] = c;
+        else if (at < cap) more[at - (uint32_t)kGCap] = c;
+    }
+};
+
+// The gathered composites [0, n) inside the packed range [lo, hi], in rank order:
 // the one where the running weight first exceeds g (excl <= g < excl + meas).  Levels
 // of kPassBins bins over the range left, until a bin holds one element.
-FIE_DEV SelResult win_select(FinSmem& S, int n, uint64_t lo, uint64_t hi, u128 g)
+FIE_DEV SelResult win_select(FinSmem& S, const WinList& wl, int n, uint64_t lo, uint64_t hi, u128 g)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     u128 excl = 0;
     // the range they span: thousands may share a key
     uint64_t mn = ~0ull, mx = 0;
     for (int i = tid; i < n; i += kFinThreads) {
-        const uint64_t c = pack_of(S.cand[i]);
+        const uint64_t c = pack_of(wl.get(S, i));
         if (c >= lo && c <= hi) {
             mn = c < mn ? c : mn;
             mx = c > mx ? c : mx;
@@ -224,11 +240,11 @@ FIE_DEV SelResult win_select(FinSmem& S, int n, uint64_t lo, uint64_t hi, u128 g
         if (tid == 0) S.ibin = -1;
         __syncthreads();
         for (int i = tid; i < n; i += kFinThreads) {
-            const uint64_t c = pack_of(S.cand[i]);
+            const uint64_t c = pack_of(wl.get(S, i));
             if (c >= lo && c <= hi) {
                 const int b = kPassBins - 1 - (int)((c - lo) >> sh);
                 atomicAdd(&S.pc[b], 1u);
-                bin_add(S, b, comp_weight(S, S.cand[i]));
+                bin_add(S, b, comp_weight(S, wl.get(S, i)));
             }
         }
         __syncthreads();
@@ -258,8 +274,8 @@ FIE_DEV SelResult win_select(FinSmem& S, int n, uint64_t lo, uint64_t hi, u128 g
         hi = top < hi ? top : hi;
         if (cnt == 1) {
             for (int i = tid; i < n; i += kFinThreads) {
-                const uint64_t c = pack_of(S.cand[i]);
-                if (c >= lo && c <= hi) S.bcomp[0] = S.cand[i];
+                const uint64_t c = pack_of(wl.get(S, i));
+                if (c >= lo && c <= hi) S.bcomp[0] = unpack_comp(c);
             }
             __syncthreads();
             const uint64_t c = S.bcomp[0];
@@ -289,9 +305,19 @@ FIE_DEV float win_y(float x, float s, float rs)
 // overflowed.  The next tile's loads are in flight while one is processed.
 enum { kWinCount, kWinSub, kWinWeigh };
 
+// A value that the optimizer does not know to equal v: it would take 32 tokens'
+// compares with v out in front of the branches that share them, and spill the results
+// (with the scheduling barriers every eight tokens, 1024 flat rows 514 -> 485 us).
+FIE_DEV float opaque(float v)
+{
+    asm("" : "+v"(v));
+    return v;
+}
+
 template <int DT>
 FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s, bool pen, float rep, float pres,
-                      float freq, float M, float y0, bool has_cut, u128& m0, u128& m1)
+                      float freq, float M, float y0, bool has_cut, const WinList& list, u128& m0,
+                      u128& m1)
 {
     constexpr int EPL = DTy<DT>::EPL, SZ = DTy<DT>::SZ, NL = kEPT / EPL;
     const fie_sampler_args& a = P.a;
@@ -348,7 +374,7 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
         const uint64_t c = pack_comp(fkey(y), idx);
         const bool in = ok && ((c >= lo0 && c <= hi0) || (has_cut && c >= lo1 && c <= hi1));
         const uint32_t at = room(in ? 1u : 0u);
-        if (in && at < (uint32_t)kWinCap) S.cand[at] = comp_key(fkey(y), idx);
+        if (in) list.put(S, at, comp_key(fkey(y), idx));
         if (ok && c > hi0) m0 += weight_of(S, y, idx);
         if (ok && has_cut && c > hi1) m1 += weight_of(S, y, idx);
     };
@@ -467,27 +493,45 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
             const float a0t = ya[0], a1t = ya[1], l0 = yl[0], u0 = yu[0], l1 = yl[1], u1 = yu[1];
             uint32_t in = 0;
             if (phase == kWinWeigh) {
-                // the weights of a lane's 32 tokens sum exactly in fp64 (below 2^46)
                 const float mt = S.mt[t + 1];
                 const uint64_t ct = S.ct[t + 1];
-                double a0 = 0.0, a1 = 0.0;
+                WeightSum s0, s1;
                 if (has_cut) {
 #pragma unroll
-                    for (int i = 0; i < kEPT; ++i) {
-                        const float wt = weight40(x[i] - mt);
-                        a0 += (double)(x[i] > a0t ? wt : 0.0f);
-                        a1 += (double)(x[i] > a1t ? wt : 0.0f);
+                    for (int i = 0; i < kEPT; i += 8) {
+                        float v0[8], v1[8];
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) {
+                            const float wt = weight20(x[i + k] - mt);
+                            v0[k] = x[i + k] > a0t ? wt : 0.0f;
+                            v1[k] = x[i + k] > a1t ? wt : 0.0f;
+                        }
+                        s0.add8(v0);
+                        s1.add8(v1);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                    m1 += (u128)(uint64_t)a1 * ct;
+                    m1 += (u128)s1.total() * ct;
                 } else {
+                    const float a0u = opaque(a0t);
 #pragma unroll
-                    for (int i = 0; i < kEPT; ++i) a0 += (double)(x[i] > a0t ? weight40(x[i] - mt) : 0.0f);
+                    for (int i = 0; i < kEPT; i += 8) {
+                        float v0[8];
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) v0[k] = x[i + k] > a0u ? weight20(x[i + k] - mt) : 0.0f;
+                        s0.add8(v0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
-                m0 += (u128)(uint64_t)a0 * ct;
+                m0 += (u128)s0.total() * ct;
             }
+            {
+                const float lo0u = opaque(l0), up0u = opaque(u0), lo1u = opaque(l1), up1u = opaque(u1);
 #pragma unroll
-            for (int i = 0; i < kEPT; ++i)
-                in |= ((x[i] >= l0 && x[i] <= u0) || (x[i] >= l1 && x[i] <= u1)) ? 1u << i : 0u;
+                for (int i = 0; i < kEPT; ++i) {
+                    if (i % 8 == 0) __builtin_amdgcn_sched_barrier(0);
+                    in |= ((x[i] >= lo0u && x[i] <= up0u) || (x[i] >= lo1u && x[i] <= up1u)) ? 1u << i : 0u;
+                }
+            }
             if (phase == kWinSub) {
                 while (__ballot(in != 0) != 0) {
                     const uint32_t i = in ? (uint32_t)__builtin_ctz(in) : 0u;
@@ -498,8 +542,7 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
                 uint32_t at = room((uint32_t)__builtin_popcount(in));
                 for (; in; in &= in - 1, ++at) {
                     const uint32_t i = (uint32_t)__builtin_ctz(in);
-                    if (at < (uint32_t)kWinCap)
-                        S.cand[at] = comp_key(fkey(pick32(x, i) + 0.0f), (uint32_t)elem_index<EPL>(lo, lane, (int)i));
+                    list.put(S, at, comp_key(fkey(pick32(x, i) + 0.0f), (uint32_t)elem_index<EPL>(lo, lane, (int)i)));
                 }
             } else {
                 // tokens equal to a window's upper end at a lower index are above it, and
@@ -512,7 +555,7 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
                     const bool ok = in != 0;
                     const bool win = ok && ((c >= lo0 && c <= hi0) || (has_cut && c >= lo1 && c <= hi1));
                     const uint32_t at = room(win ? 1u : 0u);
-                    if (win && at < (uint32_t)kWinCap) S.cand[at] = comp_key(fkey(y), idx);
+                    if (win) list.put(S, at, comp_key(fkey(y), idx));
                     if (ok && c > hi0 && !(y > a0t)) m0 += weight_of(S, y, idx);
                     if (ok && has_cut && c > hi1 && !(y > a1t)) m1 += weight_of(S, y, idx);
                     in &= in - 1;
@@ -556,8 +599,8 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
 // vocabulary.  Returns false when it decided nothing.
 template <int DT>
 FIE_DEV bool windowed_deep(FinSmem& S, const KParams& P, int row, float s, bool pen, float rep, float pres,
-                           float freq, uint32_t k0, float M, float tp, double u, u128 sall, uint64_t* cut_out,
-                           u128* T_out, uint64_t* tok_out)
+                           float freq, uint32_t k0, float M, float tp, double u, u128 sall,
+                           const WinList& list, uint64_t* cut_out, u128* T_out, uint64_t* tok_out)
 {
     const int tid = threadIdx.x, lane = tid & 63;
     if (!(s >= 0x1p-30f && s <= 0x1p30f) || !(__builtin_fabsf(M) < 0x1p40f) || sall == 0) return false;
@@ -573,7 +616,7 @@ FIE_DEV bool windowed_deep(FinSmem& S, const KParams& P, int row, float s, bool 
         if (tid == 0) S.wn = 0;
         __syncthreads();
         u128 m0 = 0, m1 = 0;
-        win_pass<DT>(S, P, row, phase, s, pen, rep, pres, freq, M, y0, has_cut, m0, m1);
+        win_pass<DT>(S, P, row, phase, s, pen, rep, pres, freq, M, y0, has_cut, list, m0, m1);
         bool lost = false;
         if (phase == kWinWeigh) {
             // the exact selections (rules R3, R4) inside the windows
@@ -582,11 +625,11 @@ FIE_DEV bool windowed_deep(FinSmem& S, const KParams& P, int row, float s, bool 
             const uint32_t n = S.wn;
             uint64_t cut = 0;
             u128 T = sall, g = 0;
-            if (n > (uint32_t)kWinCap) return false;
+            if (n > list.cap) return false;
             if (has_cut) {
                 lost = thr - 1 < m1;
                 if (!lost) {
-                    const SelResult r = win_select(S, (int)n, S.win[1].lo, S.win[1].hi, thr - 1 - m1);
+                    const SelResult r = win_select(S, list, (int)n, S.win[1].lo, S.win[1].hi, thr - 1 - m1);
                     lost = !r.found;
                     cut = r.comp;
                     T = m1 + r.excl + r.meas;
@@ -597,7 +640,7 @@ FIE_DEV bool windowed_deep(FinSmem& S, const KParams& P, int row, float s, bool 
                 lost = g < m0;
                 if (!lost) {
                     // the draw is at or above the cut: a kept token precedes every other
-                    const SelResult r = win_select(S, (int)n, S.win[0].lo, S.win[0].hi, g - m0);
+                    const SelResult r = win_select(S, list, (int)n, S.win[0].lo, S.win[0].hi, g - m0);
                     if (r.found) {
                         *cut_out = cut;
                         *T_out = T;
@@ -660,7 +703,7 @@ FIE_DEV bool windowed_deep(FinSmem& S, const KParams& P, int row, float s, bool 
             for (int k = 0; k < (has_cut ? 2 : 1); ++k) {
                 if (!((big >> k) & 1u)) continue;
                 if (phase == kWinSub && S.win[k].split) continue;
-                lost |= !win_pick(S, k, phase == kWinSub, M, k ? fc : fd, eps);
+                lost |= !win_pick(S, k, phase == kWinSub, pen, M, k ? fc : fd, eps);
             }
             __syncthreads();
             if (tid < 2) S.win[tid].split = 0;
@@ -668,8 +711,8 @@ FIE_DEV bool windowed_deep(FinSmem& S, const KParams& P, int row, float s, bool 
                 // windows with too many tokens are counted again on finer bins of the
                 // composite (the larger one first, then both)
                 const uint32_t n0 = S.win[0].n, n1 = has_cut ? S.win[1].n : 0u;
-                big = n0 + n1 <= (uint32_t)kWinCap ? 0u
-                      : (n0 > (uint32_t)kWinCap / 2 ? 1u : 0u) | (n1 > (uint32_t)kWinCap / 2 ? 2u : 0u);
+                big = n0 + n1 <= list.cap ? 0u
+                      : (n0 > list.cap / 2 ? 1u : 0u) | (n1 > list.cap / 2 ? 2u : 0u);
                 if (tid == 0) S.wbig = big;
                 if (big && ++level > 5) return false;
                 phase = big ? kWinSub : kWinWeigh;
