@@ -298,9 +298,9 @@ def cpu_baseline(w, seconds: float) -> dict:
 
 
 def time_lmhead(w, dev, H: int, steps: int = 20) -> dict:
-    """The fused lm_head (fie_sampler_lmhead_sample) against the two-step path it
-    replaces: the library GEMM torch.matmul runs for the model's output layer, then
-    fie_sampler_sample.  Same rows, parameters and histories as the headline
+    """The output layer and the sampler in one call (fie_sampler_lmhead_sample) against
+    the two-step path it replaces: the library GEMM torch.matmul runs for the model's
+    output layer, then fie_sampler_sample.  k_lmhead_us is the projection and the scan.  Same rows, parameters and histories as the headline
     workload, fp16 operands.  Hidden states and weight rows are built so the logits
     have the workload's peaked shape (-1.1 ln(rank + 1) + N(0, 0.5^2)): random
     matrices would give flat logits, and every top-p row would take the full-row path."""

@@ -4,9 +4,9 @@
 // 0's penalty, and decides the row exactly on the candidate set whenever the
 // decision provably lies among the candidates: every token whose scaled key is
 // above the largest tile bound was streamed out, so a threshold, a cut or a draw
-// that lands above that key is final.  Otherwise the row takes the full-row path
-// in the same workgroup: radix passes that re-read the row from memory, narrowing a
-// key range until it fits in LDS, then the same LDS selection.
+// that lands above that key is final.  Otherwise the row takes a full-row path, which
+// re-reads the row from memory: by windows (window.h), at once, or, with a top-k or
+// min-p threshold below the candidates, by bins and radix levels.
 #pragma once
 
 #include "scan.h"
@@ -1356,9 +1356,10 @@ FIE_DEV void sorted_find(FinSmem& S, const SortedScan& sc, u128 g, int* slot_i, 
 }
 
 // ---------------------------------------------------------------- k_finish, k_deep
-// One row's finish.  PH 0 (k_finish) settles every row its candidates can settle
-// and queues the others for PH 1 (k_deep), which runs the passes over the whole
-// row: the full-row draw, and top-L logprobs deeper than the candidates.  Both
+// One row's finish.  PH 0 (k_finish) settles every row its candidates or the windowed
+// path can settle and queues the others for PH 1 (k_deep, or the same workgroup), which
+// runs the binned passes over the whole row: thresholds below the candidates, rows with
+// span helpers, and top-L logprobs deeper than the candidates.  Both
 // phases compute the same prologue (row maximum, tile table, row mass) from the
 // partials; a queued row's DeferRec carries what PH 1 cannot recompute cheaply.
 template <int DT, int PH, int Q, bool PRE>
@@ -2107,8 +2108,8 @@ __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KPar
 }
 
 // A fixed grid taking queued rows one at a time; every workgroup leaves once the
-// queue is drained (the count is final: k_finish has completed).  The queue is
-// short in decode (a few rows a step) but holds every row of a flat batch.
+// queue is drained (the count is final: k_finish has completed).  The queue is mostly
+// empty: only thresholds or top-L logprobs below the candidates put a row there.
 template <int DT>
 __global__ __launch_bounds__(kFinThreads, 4) void k_deep(const KParams P)
 {

@@ -10,7 +10,11 @@
 //
 // The passes are laid out like k_scan's: one wave per 2048-token tile, 32 tokens a
 // lane, no barrier inside a pass.  The count is bound by its one LDS atomic a token
-// (20 cycles a wave and CU for random bins), the weighing by vector issue.
+// (21 cycles a wave and CU for random bins), the weighing by vector issue.  At vocab
+// 151936 a lone row takes 25-30 us to count, 50-75 to weigh and 10-25 to select; a step
+// of 48 open bf16 rows 194 us and one of 1024 flat rows 490, where the single weighted
+// pass it replaces (three LDS atomics and a 128-bit product a token, and radix levels
+// where a bin overflowed) took 1783 and 752.
 #pragma once
 
 // (included by finish.h, whose shared-memory layout and selections it uses)
