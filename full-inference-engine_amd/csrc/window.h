@@ -629,6 +629,13 @@ FIE_DEV bool windowed_deep(FinSmem& S, const KParams& P, int row, float s, bool 
             const uint32_t n = S.wn;
             uint64_t cut = 0;
             u128 T = sall, g = 0;
+            // A list that ran on into the candidate slots leaves the row without any, so
+            // that a finish launched again on the same partials comes here again.
+            if (n > (uint32_t)kGCap && list.cap > (uint32_t)kGCap)
+                for (int t = tid; t < P.NT; t += kFinThreads) {
+                    P.w.ncand[(size_t)row * P.NT + t] = 0;
+                    P.w.bound[(size_t)row * P.NT + t] = 0xFFFFFFFFu;
+                }
             if (n > list.cap) return false;
             if (has_cut) {
                 lost = thr - 1 < m1;

@@ -732,3 +732,44 @@ def test_helper_rows_with_shared_values(fs, dtype):
     contexts = [rng.integers(0, 60001, 200).tolist() for _ in range(12)]
     out, ref, _, _ = run_both(fs, x, params, rng.random(12), contexts, kept=False)
     check(out, ref, params)
+
+
+def _long_list_rows(rng, rows, vocab):
+    """Rows at temperature 2 whose draw mostly falls on one value, shared by 8000 tokens
+    that lie just below every tile's candidates: the tokens gathered around the draw are
+    more than the LDS list holds and run on into the row's candidate slots."""
+    x = np.full((rows, vocab), -20.0, dtype=np.float32)
+    for r in range(rows):
+        perm = rng.permutation(vocab)
+        x[r, perm[:8000]] = -3.25
+        x[r, perm[8000:11000]] = rng.uniform(-3.0, -2.4, 3000)
+        x[r, perm[-1]] = 0.0
+    return torch.from_numpy(x).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("rows", [40, 300])
+def test_finish_stage_can_be_launched_again(fs, rows):
+    """FINISH (and DEEP, for the rows it queues) launched again on the partials of one
+    SCAN gives the same outputs: what a row gathers past its LDS list must not be taken
+    for candidates."""
+    rng = np.random.default_rng(40)
+    vocab = 151936
+    x = _long_list_rows(rng, 20, vocab)
+    x = x.repeat(rows // 20, 1).to(DEV)
+    params = [SamplingParams(temperature=2.0, top_p=(1.0, 0.98)[r % 2]) for r in range(rows)]
+    u = np.tile(np.linspace(0.32, 0.46, 20), rows // 20)
+    print(f"  case: rows={rows} vocab={vocab}", flush=True)
+    out, args, buf = fs.step(x, resolve_params(params, vocab, u, None))
+    first = {k: out[k].copy() for k in ("tokens", "cut_comp", "kept_mass", "status")}
+    assert ((first["status"] & _lib.FIE_ROW_EXACT_PATH) != 0).sum() >= rows // 2
+    ref = O.canonical_step(x[:20].float().cpu().numpy(), O.resolve(params[:20], vocab), u[:20], contexts=None,
+                           want_kept=False)
+    np.testing.assert_array_equal(first["tokens"][:20], ref.tokens)
+    for again in range(2):
+        fs.launch_stage(args, _lib.FIE_STAGE_FINISH)
+        if rows > torch.cuda.get_device_properties(DEV).multi_processor_count:
+            fs.launch_stage(args, _lib.FIE_STAGE_DEEP)
+        buf.download(torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        for key, want in first.items():
+            np.testing.assert_array_equal(buf.outputs()[key], want, err_msg=f"{key}, launch {again + 2}")
