@@ -132,14 +132,17 @@ FIE_DEV float weight20(float d)
 // most 2^20.  Added, rounding down, to a float in [2^23, 2^24), whose unit is 1, each
 // part floors itself, and eight of them stay within the range: three instructions a
 // token, where a floor, a conversion to fp64 and an fp64 add took 1.5 times the cycles.
-// The rounding mode is changed and restored inside the one asm statement.
+// The rounding mode is changed and restored inside the one asm statement.  A write of the
+// mode register needs two instructions between it and the one before it, which the
+// compiler does not see inside asm: the accumulators' start values are set there.
 struct WeightSum {
     uint32_t hi = 0, lo = 0;     // sums of the float accumulators' bits, their bias removed
 
     FIE_DEV void add8(const float (&v)[8])
     {
-        float h = 0x1p23f, l = 0x1p23f, t;
-        asm("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n"
+        float h, l, t;
+        asm("v_mov_b32 %0, 0x4b000000\n v_mov_b32 %1, 0x4b000000\n"
+            "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n"
             "v_fract_f32 %2, %3\n v_add_f32 %0, %0, %3\n v_fma_f32 %1, %2, %11, %1\n"
             "v_fract_f32 %2, %4\n v_add_f32 %0, %0, %4\n v_fma_f32 %1, %2, %11, %1\n"
             "v_fract_f32 %2, %5\n v_add_f32 %0, %0, %5\n v_fma_f32 %1, %2, %11, %1\n"
@@ -149,7 +152,7 @@ struct WeightSum {
             "v_fract_f32 %2, %9\n v_add_f32 %0, %0, %9\n v_fma_f32 %1, %2, %11, %1\n"
             "v_fract_f32 %2, %10\n v_add_f32 %0, %0, %10\n v_fma_f32 %1, %2, %11, %1\n"
             "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
-            : "+&v"(h), "+&v"(l), "=&v"(t)
+            : "=&v"(h), "=&v"(l), "=&v"(t)
             : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]), "s"(0x1p20f));
         hi += __float_as_uint(h) - 0x4B000000u;
         lo += __float_as_uint(l) - 0x4B000000u;

@@ -487,3 +487,21 @@ def test_each_sampler_keeps_its_own_parameter_table():
     assert a._params(p[:1]).top_k.tolist() == [5]
     own = resolve_params(q, 100, None, None, table=tb)
     assert own.flags.tolist() == resolve_params(q, 100, None, None).flags.tolist()
+
+
+def test_mode_writes_in_asm_are_two_instructions_apart():
+    """gfx950 needs two wait states between two writes of the mode register, and the
+    compiler adds none around inline asm: a statement that writes it opens with two other
+    instructions, since a statement like it may come right before."""
+    csrc = os.path.join(os.path.dirname(_lib.__file__), "..", "csrc")
+    found = 0
+    for name in sorted(os.listdir(csrc)):
+        with open(os.path.join(csrc, name), encoding="utf-8") as f:
+            text = f.read()
+        for asm in re.findall(r'asm(?:\s+volatile)?\s*\(((?:\s*"[^"]*")+)', text):
+            lines = [i.strip() for part in re.findall(r'"([^"]*)"', asm) for i in part.split("\\n") if i.strip()]
+            writes = [i for i, ins in enumerate(lines) if ins.startswith("s_setreg")]
+            found += len(writes)
+            for at, before in zip(writes, [-1] + writes):
+                assert at - before > 2, (name, lines)
+    assert found
