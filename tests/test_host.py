@@ -527,3 +527,27 @@ def test_resolve_params_reuses_the_columns_of_an_unchanged_batch():
     with ThreadPoolExecutor(1) as ex:
         other = ex.submit(resolve_params, p, 100, None, None).result()
     assert other.scale is not mine.scale and other.scale.tolist() == mine.scale.tolist()
+
+
+def test_argmax_batches_build_no_columns():
+    """Whether a batch is all greedy, without penalties or logprobs, is asked of the objects:
+    a new batch that takes the argmax kernel pays for no column, and what the predicates say
+    is what the columns say."""
+    s = _NoKernels(generator_seed=3)
+    t = s._params([SamplingParams(), SamplingParams(temperature=0.7, top_k=1)])
+    assert t.plain and not t.wants_logprobs
+    assert not {"greedy", "lp", "shared", "own"} & set(getattr(t, "__dict__", {"greedy": 0}))
+    kinds = [dict(), dict(temperature=0.8), dict(temperature=0.8, seed=5), dict(presence_penalty=0.5),
+             dict(logprobs=0), dict(temperature=1.0, top_k=1), dict(temperature=1.0, seed=1, logprobs=3)]
+    for a in kinds:
+        for b in kinds:
+            t = s._params([SamplingParams(**a), SamplingParams(**b)])
+            assert t.plain == bool((t.greedy & ~t.pen).all())
+            assert t.wants_logprobs == bool((t.lp >= 0).any())
+            assert t.any_pen == bool(t.pen.any())
+            assert t.shared.tolist() == [r for r in (0, 1) if not t.greedy[r] and not t.seeded[r]]
+            assert t.own == [r for r in (0, 1) if not t.greedy[r] and t.seeded[r]]
+    empty = s._params([])
+    assert empty.greedy.shape == empty.seeds.shape == (0,) and empty.plain and not empty.any_pen
+    with pytest.raises(AttributeError):
+        t.unknown
