@@ -1355,14 +1355,58 @@ FIE_DEV void sorted_find(FinSmem& S, const SortedScan& sc, u128 g, int* slot_i, 
     }
 }
 
+// Queues a row for k_deep, by one thread.
+FIE_DEV void queue_row(const KParams& P, int row, const DeferRec& d)
+{
+    P.w.dfr[row] = d;
+    const uint32_t at = atomicAdd(&P.w.dq[0], 1u);
+    if (at < (uint32_t)P.a.rows) P.w.dqrows[at] = (uint32_t)row;
+}
+
+// The log of the sum of exp(y - M) over the row, from its mass; a token's logprob.
+FIE_DEV double row_lse(u128 sall) { return log(u128_to_double(sall)) - 80.0 * 0.69314718055994530942; }
+
+FIE_DEV float row_logprob(uint64_t comp, float M, double lse)
+{
+    return (float)(((double)key_to_float(comp_k(comp)) - (double)M) - lse);
+}
+
+// The row's results, by one thread.
+FIE_DEV void write_row(const KParams& P, int row, int64_t token, int32_t status, float M, uint64_t cut, u128 T, u128 sall,
+                       uint32_t tau, bool greedy, float s)
+{
+    const fie_sampler_args& a = P.a;
+    a.tokens[row] = token;
+    if (a.status) a.status[row] = status;
+    if (a.row_max) a.row_max[row] = M;
+    if (a.cut_comp) a.cut_comp[row] = cut;
+    if (greedy && a.tk_key) a.tk_key[row] = 0;
+    if (a.kept_mass) { a.kept_mass[2 * row] = (uint64_t)T; a.kept_mass[2 * row + 1] = (uint64_t)(T >> 64); }
+    if (a.row_mass) { a.row_mass[2 * row] = (uint64_t)sall; a.row_mass[2 * row + 1] = (uint64_t)(sall >> 64); }
+    RowRes rr;
+    rr.cut = cut;
+    rr.klo = (uint64_t)T;
+    rr.khi = (uint64_t)(T >> 64);
+    rr.tau = tau;
+    rr.greedy = greedy ? 1u : 0u;
+    rr.token = token;
+    rr.M = M;
+    rr.s = s;
+    P.w.res[row] = rr;
+}
+
 // ---------------------------------------------------------------- k_finish, k_deep
-// One row's finish.  PH 0 (k_finish) settles every row its candidates or the windowed
-// path can settle and queues the others for PH 1 (k_deep, or the same workgroup), which
-// runs the binned passes over the whole row: thresholds below the candidates, rows with
-// span helpers, and top-L logprobs deeper than the candidates.  Both
-// phases compute the same prologue (row maximum, tile table, row mass) from the
-// partials; a queued row's DeferRec carries what PH 1 cannot recompute cheaply.
-template <int DT, int PH, int Q, bool PRE>
+// One row's finish.  PH 0 (k_finish) settles every row its candidates can settle, takes
+// those whose cut or draw lies past them to the windowed path, and queues the others for
+// PH 1 (k_deep, or the same workgroup), which runs the binned passes over the whole row:
+// thresholds below the candidates, rows with span helpers, and top-L logprobs deeper than
+// the candidates.  Both phases compute the same prologue (row maximum, tile table, row
+// mass) from the partials; a queued row's DeferRec carries what PH 1 cannot recompute
+// cheaply.  The windowed path is part of PH 0 in the 256-register kernel (WIDE) only: in
+// 128 registers it made the whole kernel spill (156 registers; 35 without it), and rows
+// that never reach it paid (512 rows of top-k with top-p 83 us a step; 76 with the path
+// apart in window_row, and no change on the rows that do reach it).
+template <int DT, int PH, int Q, bool WIDE>
 FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool inl, const bool hd = false)
 {
     const fie_sampler_args& a = P.a;
@@ -1412,7 +1456,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     }
     // batches past the CU count are bound by traffic, and a row narrowed by mass may
     // not need its candidates at all: there they are loaded after the row mass is known
-    const bool early = spec && (PRE || !bins);
+    const bool early = spec && (WIDE || !bins);
     uint64_t xs[Q + 1];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
@@ -1560,13 +1604,11 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
             if (inl) {
                 S.dfr = d;
             } else {
-                P.w.dfr[row] = d;
-                const uint32_t at = atomicAdd(&P.w.dq[0], 1u);
-                if (at < (uint32_t)a.rows) P.w.dqrows[at] = (uint32_t)row;
+                queue_row(P, row, d);
             }
         }
     };
-    if (lp >= 0) lse = log(u128_to_double(sall)) - 80.0 * 0.69314718055994530942;
+    if (lp >= 0) lse = row_lse(sall);
 
     // Greedy rows: argmax, first index on ties (sampler.py:106,236-238).
     if (greedy) {
@@ -1725,30 +1767,64 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     // logprobs read the candidates again.
     const WinList list{P.w.cand + (size_t)row * NT * kCapW, (uint32_t)(kGCap + (lp > 0 ? 0 : NT * kCapW))};
 
-    // Full-row path for sampled rows the candidates could not settle: at once, unless
-    // the row has span helpers or a threshold whose survivors are yet to be found.
+    // Full-row path for sampled rows the candidates could not settle: by windows, at once,
+    // unless the row has span helpers or a threshold whose survivors are yet to be found.
+    bool later = false;          // window_row, after this, takes the row's cut and draw
+    const bool plain_cut = topk == 0 && !(mp > 0.0f);
+    auto windows = [&]() {
+        return windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, list, &cut, &T, &tok_comp);
+    };
     if (PH == 0 && !greedy && deep) {
-        if (P.helpers || topk > 0 || mp > 0.0f ||
-            !windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, list, &cut, &T, &tok_comp)) {
-            defer(kDeferDraw);
-            return;
+        if constexpr (WIDE) {
+            if (P.helpers || !plain_cut || !windows()) {
+                defer(kDeferDraw);
+                return;
+            }
+            status |= FIE_ROW_EXACT_PATH;
+            tau = 0;
+            token = comp_idx(tok_comp);
+            if (a.tk_key && tid == 0) a.tk_key[row] = 0;
+        } else {
+            if (!plain_cut) {
+                defer(kDeferDraw);
+                return;
+            }
+            if (tid == 0) {
+                DeferRec d{};
+                d.tlo = (uint64_t)sall;
+                d.thi = (uint64_t)(sall >> 64);
+                d.token = (int64_t)__float_as_uint(M);
+                d.tau = k0;
+                S.dfr = d;
+                S.dmode = kDeferWindows;
+            }
+            if (lp < 0) return;
+            later = true;
         }
-        status |= FIE_ROW_EXACT_PATH;
-        tau = 0;
-        token = comp_idx(tok_comp);
-        if (a.tk_key && tid == 0) a.tk_key[row] = 0;
         reload();
     }
     if (PH == 1 && !greedy && deep) {
         status |= FIE_ROW_EXACT_PATH;
-        cut = 0;
         uint32_t tk = 0;
-        const bool binned = binned_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, topk, mp, tp,
-                                                 urow, sall, &tk, &tau, &cut, &T, &tok_comp, hd);
-        // a bin too full to gather (16-bit logits share values): by windows, or
-        if (!binned && !(topk == 0 && !(mp > 0.0f) &&
-                         windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, list, &cut,
-                                           &T, &tok_comp))) {
+        bool done = false;
+        if constexpr (!WIDE) {
+            if (plain_cut && lp > 0) done = windows();      // window_row has tried the others
+        }
+        if (!done) {
+            cut = 0;
+            done = binned_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, topk, mp, tp, urow, sall, &tk, &tau, &cut,
+                                   &T, &tok_comp, hd);
+        }
+        if constexpr (WIDE) {
+            // a bin of the helpers too full to gather (16-bit logits share values); without
+            // helpers PH 0 has tried the windows
+            if (!done && hd && plain_cut) {
+                tau = 0;
+                tk = 0;
+                done = windows();
+            }
+        }
+        if (!done) {
         // radix levels over the composite, re-reading the row per level
         cut = 0;
         tk = 0;
@@ -1795,8 +1871,8 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     // Logprobs (sampler.py:262-291, rule R7): chosen token, then the row's best L,
     // all from the penalised, scaled distribution before filtering.
     if (lp >= 0) {
-        if (tid == 0 && a.chosen_logprob)
-            a.chosen_logprob[row] = (float)(((double)key_to_float(comp_k(tok_comp)) - (double)M) - lse);
+        if (tid == 0 && a.chosen_logprob && !later)
+            a.chosen_logprob[row] = row_logprob(tok_comp, M, lse);
         const int L = lp < a.lp_cols ? lp : a.lp_cols;
         if (L > 0) {
             if (sorted && nv >= L) {
@@ -1807,10 +1883,10 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
                     const uint64_t c = have ? S.cand[j] : 0ull;
                     if (a.top_ids) a.top_ids[o] = have ? (int64_t)comp_idx(c) : -1;
                     if (a.top_logprobs)
-                        a.top_logprobs[o] = have ? (float)(((double)key_to_float(comp_k(c)) - (double)M) - lse) : 0.0f;
+                        a.top_logprobs[o] = have ? row_logprob(c, M, lse) : 0.0f;
                 }
             } else if (PH == 0) {
-                defer(kDeferLogprobs);
+                defer(later ? kDeferDraw : kDeferLogprobs);
                 return;
             } else {
                 // the L-th largest composite over the row, the L composites >= it
@@ -1832,7 +1908,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
                         const bool have = j < m && j < L;
                         if (a.top_ids) a.top_ids[o] = have ? (int64_t)comp_idx(top[j]) : -1;
                         if (a.top_logprobs)
-                            a.top_logprobs[o] = have ? (float)(((double)key_to_float(comp_k(top[j])) - (double)M) - lse) : 0.0f;
+                            a.top_logprobs[o] = have ? row_logprob(top[j], M, lse) : 0.0f;
                     }
                 }
             }
@@ -1845,25 +1921,45 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         }
     }
 
+    if (PH == 0 && later) return;
     if (tid == 0) {
-        a.tokens[row] = token;
-        if (a.status) a.status[row] = status;
-        if (a.row_max) a.row_max[row] = M;
-        if (a.cut_comp) a.cut_comp[row] = cut;
-        if (greedy && a.tk_key) a.tk_key[row] = 0;
-        if (a.kept_mass) { a.kept_mass[2 * row] = (uint64_t)T; a.kept_mass[2 * row + 1] = (uint64_t)(T >> 64); }
-        if (a.row_mass) { a.row_mass[2 * row] = (uint64_t)sall; a.row_mass[2 * row + 1] = (uint64_t)(sall >> 64); }
-        RowRes rr;
-        rr.cut = cut;
-        rr.klo = (uint64_t)T;
-        rr.khi = (uint64_t)(T >> 64);
-        rr.tau = tau;
-        rr.greedy = greedy ? 1u : 0u;
-        rr.token = token;
-        rr.M = M;
-        rr.s = s;
-        P.w.res[row] = rr;
+        write_row(P, row, token, status, M, cut, T, sall, tau, greedy, s);
     }
+}
+
+// The windowed path of a row of k_finish<DT, false>, which PH 0 left with its mass,
+// maximum and token 0's key in S.dfr, its top-L logprobs written.  It reads the row's settings
+// again instead of taking them from PH 0, which would hold them in registers that rows
+// settled from their candidates need.
+template <int DT>
+FIE_DEV void window_row(FinSmem& S, const KParams& P, int row)
+{
+    asm("" : "+s"(row));        // not PH 0's row, for the optimizer
+    const fie_sampler_args& a = P.a;
+    const bool pen = a.apply_penalties && (a.flags[row] & FIE_FLAG_PENALTY);
+    const DeferRec d = S.dfr;
+    const u128 sall = ((u128)d.thi << 64) | d.tlo;
+    const float M = __uint_as_float((uint32_t)d.token), s = a.scale[row], tp = a.top_p[row];
+    float rep = 1.0f, pres = 0.0f, freq = 0.0f;
+    if (pen) { rep = a.repetition[row]; pres = a.presence[row]; freq = a.frequency[row]; }
+    const double u = a.rng ? philox_uniform(a.rng + 3 * (size_t)row) : a.uniform[row];
+    const WinList list{P.w.cand + (size_t)row * P.NT * kCapW, (uint32_t)(kGCap + P.NT * kCapW)};
+    uint64_t cut = 0, tok = 0;
+    u128 T = 0;
+    if (!windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, d.tau, M, tp, u, sall, list, &cut, &T, &tok)) {
+        if (threadIdx.x == 0) {
+            DeferRec q{};
+            q.mode = kDeferDraw;
+            queue_row(P, row, q);
+        }
+        return;
+    }
+    if (threadIdx.x != 0) return;
+    const int lp = a.logprobs ? a.logprobs[row] : -1;
+    if (lp >= 0 && a.chosen_logprob) a.chosen_logprob[row] = row_logprob(tok, M, row_lse(sall));
+    if (a.tk_key) a.tk_key[row] = 0;
+    const int32_t status = FIE_ROW_EXACT_PATH | (pen && P.w.bad[row] && !a.hist_invalid ? FIE_ROW_UNCOUNTED_IDS : 0);
+    write_row(P, row, comp_idx(tok), status, M, cut, T, sall, 0u, false, s);
 }
 
 // ---------------------------------------------------------------- span helpers
@@ -2076,8 +2172,8 @@ FIE_DEV bool span_helper(FinSmem& S, const KParams& P, const int row, const int 
 
 // One workgroup per row.  A row's finish is a chain of dependent steps, so its
 // latency is the kernel's: with no more rows than CUs (one workgroup each) the WIDE
-// variant takes up to 256 registers a lane and spills nothing; larger batches take
-// 128 (two workgroups a CU).
+// variant takes up to 256 registers a lane (12 spilled, in the full-row paths); larger
+// batches take 128 (two workgroups a CU).
 template <int DT, bool WIDE>
 __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KParams P)
 {
@@ -2101,15 +2197,17 @@ __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KPar
                 hd = true;
             }
         }
-        if (deep) finish_row<DT, 1, kReloadQ, false>(S, P, blockIdx.x, inl, hd);
+        if (deep) finish_row<DT, 1, kReloadQ, true>(S, P, blockIdx.x, inl, hd);
     } else {
         finish_row<DT, 0, kReloadQ, false>(S, P, blockIdx.x, false);
+        __syncthreads();
+        if (S.dmode == kDeferWindows) window_row<DT>(S, P, blockIdx.x);
     }
 }
 
-// A fixed grid taking queued rows one at a time; every workgroup leaves once the
-// queue is drained (the count is final: k_finish has completed).  The queue is mostly
-// empty: only thresholds or top-L logprobs below the candidates put a row there.
+// One workgroup per queue entry; those past the queued count leave at once (the count is
+// final: k_finish has completed).  The queue is mostly empty: only thresholds or top-L
+// logprobs below the candidates put a row there.
 template <int DT>
 __global__ __launch_bounds__(kFinThreads, 4) void k_deep(const KParams P)
 {
@@ -2117,7 +2215,13 @@ __global__ __launch_bounds__(kFinThreads, 4) void k_deep(const KParams P)
     const uint32_t queued = P.w.dq[0];
     const uint32_t total = queued < (uint32_t)P.a.rows ? queued : (uint32_t)P.a.rows;
     if (blockIdx.x >= total) return;
-    finish_row<DT, 1, kReloadQ, false>(S, P, (int)P.w.dqrows[blockIdx.x], false);
+    // k_finish launched again on one scan's partials queues its rows again: the first
+    // entry settles a row, for two workgroups would share its list
+    const uint32_t row = P.w.dqrows[blockIdx.x];
+    bool again = false;
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kFinThreads) again |= P.w.dqrows[i] == row;
+    if (__syncthreads_or(again)) return;
+    finish_row<DT, 1, kReloadQ, false>(S, P, (int)row, false);
 }
 
 }  // namespace fie

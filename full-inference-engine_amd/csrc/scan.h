@@ -54,7 +54,9 @@ struct RowRes {
 // A row k_finish hands to k_deep: what the full-row passes need beyond what k_deep
 // recomputes from the partials (mode kDeferDraw), or that the candidates settled
 // the draw and only the top-L logprobs need a pass over the row (kDeferLogprobs).
-constexpr uint32_t kDeferDraw = 1, kDeferLogprobs = 2;
+// kDeferWindows: the row goes on to window_row in the same workgroup, its mass in tlo and
+// thi, its maximum's bits in token, token 0's key in tau.
+constexpr uint32_t kDeferDraw = 1, kDeferLogprobs = 2, kDeferWindows = 3;
 struct DeferRec {
     uint64_t tok_comp, cut, tlo, thi;
     int64_t token;

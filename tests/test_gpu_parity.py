@@ -773,3 +773,37 @@ def test_finish_stage_can_be_launched_again(fs, rows):
         torch.cuda.synchronize()
         for key, want in first.items():
             np.testing.assert_array_equal(buf.outputs()[key], want, err_msg=f"{key}, launch {again + 2}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_rows_of_batches_past_the_cu_count(fs, dtype):
+    """The per-row kernel of batches past the CU count: rows settled from their candidates,
+    rows it takes by windows after (top-p and plain draws, with and without penalties, with
+    top-L logprobs from the candidates), and rows it queues (thresholds below the candidates,
+    logprobs below them on rows of one value).  FINISH and DEEP launched again on the same
+    partials queue those rows twice and give the same outputs."""
+    rng = np.random.default_rng(300)
+    rows, vocab = 300, 20011
+    x = torch.cat([_deep_rows(rng, rows // 3, vocab, dtype, kind) for kind in ("flat", "peaked", "constant")])
+    pen = dict(repetition_penalty=1.2, frequency_penalty=0.3, presence_penalty=0.1)
+    kinds = [dict(temperature=1.0, top_p=0.95), dict(temperature=0.8, top_p=0.9, **pen), dict(temperature=1.0),
+             dict(temperature=1.0, top_p=0.97, logprobs=0), dict(temperature=1.1, top_p=0.99, logprobs=5, **pen),
+             dict(temperature=1.0, logprobs=20), dict(temperature=1.0, top_k=3000, top_p=0.9, **pen),
+             dict(temperature=1.0, min_p=0.3, **pen), dict(temperature=0.7, top_k=40, logprobs=3), dict(logprobs=20, **pen)]
+    params = [SamplingParams(**kinds[r % len(kinds)]) for r in range(rows)]
+    ctx = [rng.integers(0, vocab, 300).tolist() + [8200] * (700 if r % 20 == 1 else 0) for r in range(rows)]
+    u = rng.random(rows)
+    hp = resolve_params(params, vocab, u, ctx)
+    print(f"  case: rows={rows} vocab={vocab} dtype={dtype}", flush=True)
+    out, args, buf = fs.step(x.to(DEV), hp)
+    first = {k: v.copy() for k, v in out.items()}
+    ref = O.canonical_step(x.float().numpy(), O.resolve(params, vocab), u, contexts=ctx, want_kept=False)
+    check(first, ref, params, lp=True)
+    assert ((first["status"] & _lib.FIE_ROW_EXACT_PATH) != 0).sum() > rows // 3
+    for again in range(2):
+        fs.launch_stage(args, _lib.FIE_STAGE_FINISH)
+        fs.launch_stage(args, _lib.FIE_STAGE_DEEP)
+        buf.download(torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        for key, want in first.items():
+            np.testing.assert_array_equal(buf.outputs()[key], want, err_msg=f"{key}, launch {again + 2}")
