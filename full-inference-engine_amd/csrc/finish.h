@@ -1371,6 +1371,9 @@ FIE_DEV float row_logprob(uint64_t comp, float M, double lse)
     return (float)(((double)key_to_float(comp_k(comp)) - (double)M) - lse);
 }
 
+// Whether no threshold restricts a sampled row but its top-p cut.
+FIE_DEV bool plain_cut(int topk, float mp) { return topk == 0 && !(mp > 0.0f); }
+
 // The row's results, by one thread.
 FIE_DEV void write_row(const KParams& P, int row, int64_t token, int32_t status, float M, uint64_t cut, u128 T, u128 sall,
                        uint32_t tau, bool greedy, float s)
@@ -1396,18 +1399,16 @@ FIE_DEV void write_row(const KParams& P, int row, int64_t token, int32_t status,
 }
 
 // ---------------------------------------------------------------- k_finish, k_deep
-// One row's finish.  PH 0 (k_finish) settles every row its candidates can settle, takes
-// those whose cut or draw lies past them to the windowed path, and queues the others for
-// PH 1 (k_deep, or the same workgroup), which runs the binned passes over the whole row:
-// thresholds below the candidates, rows with span helpers, and top-L logprobs deeper than
-// the candidates.  Both phases compute the same prologue (row maximum, tile table, row
-// mass) from the partials; a queued row's DeferRec carries what PH 1 cannot recompute
-// cheaply.  The windowed path is part of PH 0 in the 256-register kernel (WIDE) only: in
-// 128 registers it made the whole kernel spill (156 registers; 35 without it), and rows
-// that never reach it paid (512 rows of top-k with top-p 83 us a step; 76 with the path
-// apart in window_row, and no change on the rows that do reach it).
-template <int DT, int PH, int Q, bool WIDE>
-FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool inl, const bool hd = false)
+// One row's finish: settled where its candidates can settle it.  A row whose cut, draw
+// or threshold lies past them goes on to the full-row paths (window_row, binned_row,
+// radix_row), its record in S.dfr and the next of them in S.dmode; its top-L logprobs are
+// written here all the same, or left to radix_row where they are deeper than its
+// candidates.  The windowed path is part of this function in the 256-register kernel
+// (WIDE) only: in 128 registers it made the whole kernel spill (156 registers; 35 without
+// it), and rows that never reach it paid (512 rows of top-k with top-p 83 us a step; 76
+// with the path apart in window_row, and no change on the rows that do reach it).
+template <int DT, int Q, bool WIDE>
+FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row)
 {
     const fie_sampler_args& a = P.a;
     const int tid = threadIdx.x, NT = P.NT;
@@ -1428,8 +1429,8 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     if (pen && P.w.bad[row] && !a.hist_invalid) status |= FIE_ROW_UNCOUNTED_IDS;
 
     // Every per-tile partial this row reads, loaded together up front: the tile
-    // maxima, sums, candidate counts and bounds, token 0's logit and count, and in
-    // PH 0 the candidate slots of the first kFinWaves * Q tiles (a tile's count
+    // maxima, sums, candidate counts and bounds, token 0's logit and count, and
+    // the candidate slots of the first kFinWaves * Q tiles (a tile's count
     // arrives with them, so all its slots are read and the invalid ones dropped).
     const bool need_cand = !greedy || lp > 0;
     const int lane = tid & 63, wave = tid >> 6;
@@ -1440,7 +1441,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     const uint32_t pf_bd = (need_cand && tid < NT) ? P.w.bound[tbase] : 0u;
     const float x0 = P.w.tok0x[row];
     const uint32_t c0 = pen ? P.w.tok0c[row] : 0u;
-    const bool spec = PH == 0 && need_cand;
+    const bool spec = need_cand;
     // rows narrowed by mass (no top-k, no min-p) bin their candidates as they are taken
     const bool bins = spec && !greedy && topk == 0 && !(mp > 0.0f);
     // rows narrowed by count (top-k, top-L) whose every tile's slots are held in
@@ -1476,7 +1477,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         if (tid == 0) {
             S.n = 0;
             S.cmax = 0;
-            if (PH == 0) S.dmode = 0;            // PH 1 in place: the caller has read it
+            S.dmode = 0;
         }
     }
     __syncthreads();
@@ -1533,7 +1534,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     else if (kx > kKeyPosInf) safe = 0xFFFFFFFFu;
     else safe = fkey(y_of_xkey(kx, s));
 
-    // PH 0: the candidates as y-domain composites, those above the safety key into
+    // The candidates as y-domain composites, those above the safety key into
     // S.cand (binned when narrowed by mass); tiles past the held ones load now.
     bool okr[Q + 1];             // the held slots, for the second sweep
     auto commit = [&]() {
@@ -1586,28 +1587,6 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     u128 T = 0;
     bool deep = false;
     double lse = 0.0;
-    DeferRec dr{};
-    if (PH == 1) dr = inl ? S.dfr : P.w.dfr[row];
-    // PH 0: hand the row to the full-row path with what is settled so far: in place
-    // (inl: the caller runs PH 1 next, the record in LDS) or queued for k_deep
-    auto defer = [&](uint32_t mode) {
-        if (tid == 0) {
-            DeferRec d;
-            d.tok_comp = tok_comp;
-            d.cut = cut;
-            d.tlo = (uint64_t)T;
-            d.thi = (uint64_t)(T >> 64);
-            d.token = token;
-            d.tau = tau;
-            d.mode = mode;
-            S.dmode = mode;
-            if (inl) {
-                S.dfr = d;
-            } else {
-                queue_row(P, row, d);
-            }
-        }
-    };
     if (lp >= 0) lse = row_lse(sall);
 
     // Greedy rows: argmax, first index on ties (sampler.py:106,236-238).
@@ -1626,13 +1605,8 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
     uint64_t cmax = 0;       // the largest candidate composite
     bool sorted = false;
     if (need_cand) {
-        if (PH == 1) {
-            // the row was queued: its candidates are reloaded below only for logprobs
-            deep = dr.mode == kDeferDraw;
-        } else {
         nv = (int)S.n;
         cmax = S.cmax;
-
 
         if (far || nv > kSortMax) {
             deep = true;
@@ -1684,21 +1658,12 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
                 sorted = true;
             }
         }
-        }
     }
-    if (PH == 1 && dr.mode == kDeferLogprobs) {
-        token = dr.token;
-        tok_comp = dr.tok_comp;
-        tau = dr.tau;
-        cut = dr.cut;
-        T = ((u128)dr.thi << 64) | dr.tlo;
-    }
-
     // Sampled rows on the sorted candidates: top-k, min-p, S, top-p cut, draw.  The
     // narrowed prefix holds every crossing by construction; should a cut or draw
     // still miss it, that is not a verdict: every candidate is then loaded and
     // sorted and the selection runs again.
-    if (PH == 0 && !greedy && !deep) {
+    if (!greedy && !deep) {
         for (;;) {
             const bool partial = nv < nvall;
             bool miss = false;
@@ -1763,78 +1728,201 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
         }
     };
 
-    // The windowed path's list may run on into the row's candidate slots unless the
-    // logprobs read the candidates again.
-    const WinList list{P.w.cand + (size_t)row * NT * kCapW, (uint32_t)(kGCap + (lp > 0 ? 0 : NT * kCapW))};
-
-    // Full-row path for sampled rows the candidates could not settle: by windows, at once,
-    // unless the row has span helpers or a threshold whose survivors are yet to be found.
-    bool later = false;          // window_row, after this, takes the row's cut and draw
-    const bool plain_cut = topk == 0 && !(mp > 0.0f);
-    auto windows = [&]() {
-        return windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, list, &cut, &T, &tok_comp);
-    };
-    if (PH == 0 && !greedy && deep) {
+    // Rows the candidates could not settle: without a threshold below them by windows first,
+    // in place where there are no span helpers; the others by bins.  (Greedy rows always
+    // settle.)
+    uint32_t next = 0;
+    if (deep) {
+        const bool plain = plain_cut(topk, mp);
+        next = plain && !P.helpers ? kDeferWindows : kDeferDraw;
         if constexpr (WIDE) {
-            if (P.helpers || !plain_cut || !windows()) {
-                defer(kDeferDraw);
-                return;
+            if (next == kDeferWindows) {
+                // the list may run on into the candidate slots unless the logprobs read them again
+                const WinList list{P.w.cand + (size_t)row * NT * kCapW, (uint32_t)(kGCap + (lp > 0 ? 0 : NT * kCapW))};
+                next = kDeferDraw;
+                if (windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, list, &cut, &T, &tok_comp)) {
+                    next = 0;
+                    status |= FIE_ROW_EXACT_PATH;
+                    tau = 0;
+                    token = comp_idx(tok_comp);
+                    if (a.tk_key && tid == 0) a.tk_key[row] = 0;
+                }
             }
-            status |= FIE_ROW_EXACT_PATH;
-            tau = 0;
-            token = comp_idx(tok_comp);
-            if (a.tk_key && tid == 0) a.tk_key[row] = 0;
-        } else {
-            if (!plain_cut) {
-                defer(kDeferDraw);
-                return;
-            }
-            if (tid == 0) {
-                DeferRec d{};
-                d.tlo = (uint64_t)sall;
-                d.thi = (uint64_t)(sall >> 64);
-                d.token = (int64_t)__float_as_uint(M);
-                d.tau = k0;
-                S.dfr = d;
-                S.dmode = kDeferWindows;
-            }
-            if (lp < 0) return;
-            later = true;
         }
-        reload();
+        // the LDS candidates again, for the logprobs
+        sorted = false;
+        if (lp > 0) {
+            nv = load_candidates(S, P, row, NT, s, k0, safe);
+            if (nv <= kSortMax) {
+                sort_desc(S, nv);
+                sorted = true;
+            }
+        }
     }
-    if (PH == 1 && !greedy && deep) {
-        status |= FIE_ROW_EXACT_PATH;
-        uint32_t tk = 0;
-        bool done = false;
-        if constexpr (!WIDE) {
-            if (plain_cut && lp > 0) done = windows();      // window_row has tried the others
-        }
-        if (!done) {
-            cut = 0;
-            done = binned_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, topk, mp, tp, urow, sall, &tk, &tau, &cut,
-                                   &T, &tok_comp, hd);
-        }
-        if constexpr (WIDE) {
-            // a bin of the helpers too full to gather (16-bit logits share values); without
-            // helpers PH 0 has tried the windows
-            if (!done && hd && plain_cut) {
-                tau = 0;
-                tk = 0;
-                done = windows();
+
+    // Logprobs (sampler.py:262-291, rule R7): chosen token, then the row's best L,
+    // all from the penalised, scaled distribution before filtering.
+    bool needl = false;
+    if (lp >= 0) {
+        if (tid == 0 && a.chosen_logprob && !next) a.chosen_logprob[row] = row_logprob(tok_comp, M, lse);
+        const int L = lp < a.lp_cols ? lp : a.lp_cols;
+        needl = L > 0 && !(sorted && nv >= L);
+        if (!needl) {
+            // the first L sorted candidates
+            for (int j = tid; j < a.lp_cols; j += kFinThreads) {
+                const size_t o = (size_t)row * a.lp_cols + j;
+                const bool have = j < L;
+                const uint64_t c = have ? S.cand[j] : 0ull;
+                if (a.top_ids) a.top_ids[o] = have ? (int64_t)comp_idx(c) : -1;
+                if (a.top_logprobs) a.top_logprobs[o] = have ? row_logprob(c, M, lse) : 0.0f;
             }
         }
-        if (!done) {
-        // radix levels over the composite, re-reading the row per level
-        cut = 0;
-        tk = 0;
-        if (topk > 0) {
-            const SelResult r = row_select<DT, false>(S, P, row, s, pen, rep, pres, freq, k0,
-                                                           Pred{0, 0, 0}, (u128)(topk - 1), false);
-            tk = comp_k(r.comp);
+    }
+
+    if (tid != 0) return;
+    if (next == 0 && !needl) {
+        write_row(P, row, token, status, M, cut, T, sall, tau, greedy, s);
+        return;
+    }
+    DeferRec d;
+    d.tok_comp = tok_comp;
+    d.cut = cut;
+    d.T = T;
+    d.sall = sall;
+    d.token = token;
+    d.tau = tau;
+    d.k0 = k0;
+    d.M = M;
+    d.status = status;
+    d.needl = needl ? 1u : 0u;
+    d.mode = next ? next : kDeferLogprobs;
+    if (WIDE || next == kDeferWindows) {
+        S.dfr = d;
+        S.dmode = d.mode;
+    } else {
+        queue_row(P, row, d);
+    }
+}
+
+// A row's settings, read again by the full-row paths: taken from finish_row they would be
+// held there in registers that rows settled from their candidates need.
+struct RowSet {
+    bool pen;
+    float s, rep, pres, freq, tp, mp;
+    int topk;
+    double u;
+};
+
+FIE_DEV RowSet row_settings(const KParams& P, int row)
+{
+    // every load at once, then what applies
+    const fie_sampler_args& a = P.a;
+    RowSet r{false, a.scale[row], 1.0f, 0.0f, 0.0f, a.top_p[row], a.min_p[row], a.top_k[row], 0.0};
+    const int32_t fl = a.flags[row];
+    if (a.apply_penalties) {
+        const float rep = a.repetition[row], pres = a.presence[row], freq = a.frequency[row];
+        r.pen = fl & FIE_FLAG_PENALTY;
+        if (r.pen) { r.rep = rep; r.pres = pres; r.freq = freq; }
+    }
+    r.u = a.rng ? philox_uniform(a.rng + 3 * (size_t)row) : a.uniform[row];
+    if (fl & FIE_FLAG_GREEDY) { r.s = 1.0f; r.tp = 1.0f; r.mp = 0.0f; r.topk = 0; }
+    return r;
+}
+
+// A draw settled by a full-row path, by one thread: the row is written, or goes on to its
+// top-L logprobs.  Returns the next mode.
+FIE_DEV uint32_t settle_row(FinSmem& S, const KParams& P, int row, float s, uint64_t tok, uint32_t tk, uint32_t tau,
+                            uint64_t cut, u128 T)
+{
+    const fie_sampler_args& a = P.a;
+    DeferRec& d = S.dfr;
+    if (a.logprobs && a.logprobs[row] >= 0 && a.chosen_logprob) a.chosen_logprob[row] = row_logprob(tok, d.M, row_lse(d.sall));
+    if (a.tk_key) a.tk_key[row] = tk;
+    d.status |= FIE_ROW_EXACT_PATH;
+    if (!d.needl) {
+        write_row(P, row, comp_idx(tok), d.status, d.M, cut, T, d.sall, tau, false, s);
+        return 0;
+    }
+    d.tok_comp = tok;
+    d.token = comp_idx(tok);
+    d.tau = tau;
+    d.cut = cut;
+    d.T = T;
+    return kDeferLogprobs;
+}
+
+// The full-row paths, each a function of its own: compiled together the windowed and the
+// binned passes took 10% longer (20 flat rows with min-p 363 us a step; 339 apart).  Each
+// reads its row's record in S.dfr and leaves in S.dmode what is still to be done.
+template <int DT>
+FIE_DEV void window_row(FinSmem& S, const KParams& P, int row, const bool hd)
+{
+    asm("" : "+s"(row));        // not finish_row's row, for the optimizer
+    const fie_sampler_args& a = P.a;
+    RowSet r;                   // never a greedy row: what the windows need, and no more
+    r.pen = a.apply_penalties && (a.flags[row] & FIE_FLAG_PENALTY);
+    r.s = a.scale[row];
+    r.tp = a.top_p[row];
+    r.rep = 1.0f;
+    r.pres = r.freq = 0.0f;
+    if (r.pen) { r.rep = a.repetition[row]; r.pres = a.presence[row]; r.freq = a.frequency[row]; }
+    r.u = a.rng ? philox_uniform(a.rng + 3 * (size_t)row) : a.uniform[row];
+    const u128 sall = S.dfr.sall;
+    const float M = S.dfr.M;
+    const uint32_t k0 = S.dfr.k0;
+    const WinList list{P.w.cand + (size_t)row * P.NT * kCapW, (uint32_t)(kGCap + P.NT * kCapW)};
+    uint64_t cut = 0, tok = 0;
+    u128 T = 0;
+    const bool done = windowed_deep<DT>(S, P, row, r.s, r.pen, r.rep, r.pres, r.freq, k0, M, r.tp, r.u, sall, list, &cut,
+                                        &T, &tok);
+    __syncthreads();                // every thread has read S.dmode and S.dfr
+    if (threadIdx.x == 0)           // (hd: the helpers' bins did not do)
+        S.dmode = done ? settle_row(S, P, row, r.s, tok, 0u, 0u, cut, T) : (hd ? kDeferRadix : kDeferDraw);
+}
+
+template <int DT>
+FIE_DEV void binned_row(FinSmem& S, const KParams& P, int row, const bool hd)
+{
+    asm("" : "+s"(row));
+    const RowSet r = row_settings(P, row);
+    const u128 sall = S.dfr.sall;
+    const float M = S.dfr.M;
+    const uint32_t k0 = S.dfr.k0;
+    uint64_t cut = 0, tok = 0;
+    uint32_t tk = 0, tau = 0;
+    u128 T = 0;
+    const bool done = binned_deep<DT>(S, P, row, r.s, r.pen, r.rep, r.pres, r.freq, k0, M, r.topk, r.mp, r.tp, r.u, sall,
+                                      &tk, &tau, &cut, &T, &tok, hd);
+    __syncthreads();                // every thread has read S.dmode and S.dfr
+    if (threadIdx.x == 0)
+        // a bin of the helpers too full to gather (16-bit logits share values): by windows
+        S.dmode = done ? settle_row(S, P, row, r.s, tok, tk, tau, cut, T)
+                       : (hd && plain_cut(r.topk, r.mp) ? kDeferWindows : kDeferRadix);
+}
+
+// What is left: the draw by radix levels over the composite, re-reading the row per level
+// (kDeferRadix), then the top-L logprobs that the candidates did not hold.
+template <int DT>
+FIE_DEV void radix_row(FinSmem& S, const KParams& P, int row)
+{
+    asm("" : "+s"(row));
+    const fie_sampler_args& a = P.a;
+    const RowSet r = row_settings(P, row);
+    const int tid = threadIdx.x;
+    const float s = r.s, rep = r.rep, pres = r.pres, freq = r.freq, M = S.dfr.M;
+    const bool pen = r.pen;
+    const uint32_t k0 = S.dfr.k0;
+    if (S.dmode == kDeferRadix) {
+        uint64_t cut = 0, tok = 0;
+        uint32_t tk = 0;
+        u128 T;
+        if (r.topk > 0) {
+            const SelResult q = row_select<DT, false>(S, P, row, s, pen, rep, pres, freq, k0, Pred{0, 0, 0},
+                                                      (u128)(r.topk - 1), false);
+            tk = comp_k(q.comp);
         }
-        const uint32_t tmp = minp_key(M, mp);
-        tau = tk > tmp ? tk : tmp;
+        const uint32_t tmp = minp_key(M, r.mp);
+        const uint32_t tau = tk > tmp ? tk : tmp;
         const Pred surv{tau, 0, 0};
         pass_hist<DT, true>(S, P, row, s, pen, rep, pres, freq, k0, surv, 0, 0);
         u128 part = 0;
@@ -1842,124 +1930,63 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row, const bool 
             part += ((u128)S.pm_hi[b] << 64) | S.pm_lo[b];
         const u128 Sv = block_sum_u128<kFinThreads>(part, S.red128);
         bool l1 = true;
-        if (tp < 1.0f) {
-            const u128 thr = ceil_mul_f32(tp, Sv);
-            const SelResult r = row_select<DT, true>(S, P, row, s, pen, rep, pres, freq, k0,
-                                                          surv, thr - 1, true);
-            cut = r.comp;
-            T = r.excl + r.meas;
+        if (r.tp < 1.0f) {
+            const u128 thr = ceil_mul_f32(r.tp, Sv);
+            const SelResult q = row_select<DT, true>(S, P, row, s, pen, rep, pres, freq, k0, surv, thr - 1, true);
+            cut = q.comp;
+            T = q.excl + q.meas;
             l1 = false;
         } else {
             T = Sv;
         }
         if (T == 0) {
-            const SelResult r = row_select<DT, false>(S, P, row, s, pen, rep, pres, freq, k0,
-                                                           Pred{0, 0, 0}, 0, false);
-            tok_comp = r.comp;
+            tok = row_select<DT, false>(S, P, row, s, pen, rep, pres, freq, k0, Pred{0, 0, 0}, 0, false).comp;
         } else {
-            const u128 g = floor_mul_f64(urow, T);
-            const SelResult r = row_select<DT, true>(S, P, row, s, pen, rep, pres, freq, k0,
-                                                          Pred{tau, 0, cut}, g, l1);
-            tok_comp = r.comp;
+            const u128 g = floor_mul_f64(r.u, T);
+            tok = row_select<DT, true>(S, P, row, s, pen, rep, pres, freq, k0, Pred{tau, 0, cut}, g, l1).comp;
         }
-        }
-        token = comp_idx(tok_comp);
-        if (a.tk_key && tid == 0) a.tk_key[row] = tk;
-        reload();
+        if (tid == 0) settle_row(S, P, row, s, tok, tk, tau, cut, T);
+        __syncthreads();
     }
-
-    // Logprobs (sampler.py:262-291, rule R7): chosen token, then the row's best L,
-    // all from the penalised, scaled distribution before filtering.
-    if (lp >= 0) {
-        if (tid == 0 && a.chosen_logprob && !later)
-            a.chosen_logprob[row] = row_logprob(tok_comp, M, lse);
-        const int L = lp < a.lp_cols ? lp : a.lp_cols;
-        if (L > 0) {
-            if (sorted && nv >= L) {
-                // the first L sorted candidates
-                for (int j = tid; j < a.lp_cols; j += kFinThreads) {
-                    const size_t o = (size_t)row * a.lp_cols + j;
-                    const bool have = j < L;
-                    const uint64_t c = have ? S.cand[j] : 0ull;
-                    if (a.top_ids) a.top_ids[o] = have ? (int64_t)comp_idx(c) : -1;
-                    if (a.top_logprobs)
-                        a.top_logprobs[o] = have ? row_logprob(c, M, lse) : 0.0f;
-                }
-            } else if (PH == 0) {
-                defer(later ? kDeferDraw : kDeferLogprobs);
-                return;
-            } else {
-                // the L-th largest composite over the row, the L composites >= it
-                // gathered, then sorted by one thread
-                const SelResult r = row_select<DT, false>(S, P, row, s, pen, rep, pres, freq, k0,
-                                                               Pred{0, 0, 0}, (u128)(L - 1), false);
-                n = pass_gather<DT>(S, P, row, s, pen, rep, pres, freq, k0, Pred{0, 0, r.comp}, 64, 0);
-                if (tid == 0) {
-                    const int m = n < 32 ? n : 32;
-                    uint64_t* top = S.cand;
-                    for (int i = 1; i < m; ++i) {
-                        const uint64_t c = top[i];
-                        int j = i;
-                        while (j > 0 && top[j - 1] < c) { top[j] = top[j - 1]; --j; }
-                        top[j] = c;
-                    }
-                    for (int j = 0; j < a.lp_cols; ++j) {
-                        const size_t o = (size_t)row * a.lp_cols + j;
-                        const bool have = j < m && j < L;
-                        if (a.top_ids) a.top_ids[o] = have ? (int64_t)comp_idx(top[j]) : -1;
-                        if (a.top_logprobs)
-                            a.top_logprobs[o] = have ? row_logprob(top[j], M, lse) : 0.0f;
-                    }
-                }
-            }
-        } else if (tid == 0) {
-            for (int j = 0; j < a.lp_cols; ++j) {
-                const size_t o = (size_t)row * a.lp_cols + j;
-                if (a.top_ids) a.top_ids[o] = -1;
-                if (a.top_logprobs) a.top_logprobs[o] = 0.0f;
-            }
-        }
+    if (!S.dfr.needl) return;
+    // the L-th largest composite over the row, the L composites >= it gathered, then
+    // sorted by one thread
+    const int L = min(a.logprobs[row], a.lp_cols);
+    const SelResult q = row_select<DT, false>(S, P, row, s, pen, rep, pres, freq, k0, Pred{0, 0, 0}, (u128)(L - 1), false);
+    const int n = pass_gather<DT>(S, P, row, s, pen, rep, pres, freq, k0, Pred{0, 0, q.comp}, 64, 0);
+    if (tid != 0) return;
+    const DeferRec& d = S.dfr;
+    const double lse = row_lse(d.sall);
+    const int m = n < 32 ? n : 32;
+    uint64_t* top = S.cand;
+    for (int i = 1; i < m; ++i) {
+        const uint64_t c = top[i];
+        int j = i;
+        while (j > 0 && top[j - 1] < c) { top[j] = top[j - 1]; --j; }
+        top[j] = c;
     }
-
-    if (PH == 0 && later) return;
-    if (tid == 0) {
-        write_row(P, row, token, status, M, cut, T, sall, tau, greedy, s);
+    for (int j = 0; j < a.lp_cols; ++j) {
+        const size_t o = (size_t)row * a.lp_cols + j;
+        const bool have = j < m && j < L;
+        if (a.top_ids) a.top_ids[o] = have ? (int64_t)comp_idx(top[j]) : -1;
+        if (a.top_logprobs) a.top_logprobs[o] = have ? row_logprob(top[j], M, lse) : 0.0f;
     }
+    write_row(P, row, d.token, d.status, M, d.cut, d.T, d.sall, d.tau, a.flags[row] & FIE_FLAG_GREEDY, s);
 }
 
-// The windowed path of a row of k_finish<DT, false>, which PH 0 left with its mass,
-// maximum and token 0's key in S.dfr, its top-L logprobs written.  It reads the row's settings
-// again instead of taking them from PH 0, which would hold them in registers that rows
-// settled from their candidates need.
-template <int DT>
-FIE_DEV void window_row(FinSmem& S, const KParams& P, int row)
+// A row handed over from another workgroup: its record and its tile table into LDS.
+FIE_DEV void take_row(FinSmem& S, const KParams& P, int row)
 {
-    asm("" : "+s"(row));        // not PH 0's row, for the optimizer
-    const fie_sampler_args& a = P.a;
-    const bool pen = a.apply_penalties && (a.flags[row] & FIE_FLAG_PENALTY);
-    const DeferRec d = S.dfr;
-    const u128 sall = ((u128)d.thi << 64) | d.tlo;
-    const float M = __uint_as_float((uint32_t)d.token), s = a.scale[row], tp = a.top_p[row];
-    float rep = 1.0f, pres = 0.0f, freq = 0.0f;
-    if (pen) { rep = a.repetition[row]; pres = a.presence[row]; freq = a.frequency[row]; }
-    const double u = a.rng ? philox_uniform(a.rng + 3 * (size_t)row) : a.uniform[row];
-    const WinList list{P.w.cand + (size_t)row * P.NT * kCapW, (uint32_t)(kGCap + P.NT * kCapW)};
-    uint64_t cut = 0, tok = 0;
-    u128 T = 0;
-    if (!windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, d.tau, M, tp, u, sall, list, &cut, &T, &tok)) {
-        if (threadIdx.x == 0) {
-            DeferRec q{};
-            q.mode = kDeferDraw;
-            queue_row(P, row, q);
-        }
-        return;
+    const size_t base = (size_t)row * (P.NT + 1);
+    for (int i = threadIdx.x; i <= P.NT; i += kFinThreads) {
+        S.mt[i] = P.w.mt[base + i];
+        S.ct[i] = P.w.ct[base + i];
     }
-    if (threadIdx.x != 0) return;
-    const int lp = a.logprobs ? a.logprobs[row] : -1;
-    if (lp >= 0 && a.chosen_logprob) a.chosen_logprob[row] = row_logprob(tok, M, row_lse(sall));
-    if (a.tk_key) a.tk_key[row] = 0;
-    const int32_t status = FIE_ROW_EXACT_PATH | (pen && P.w.bad[row] && !a.hist_invalid ? FIE_ROW_UNCOUNTED_IDS : 0);
-    write_row(P, row, comp_idx(tok), status, M, cut, T, sall, 0u, false, s);
+    if (threadIdx.x == 0) {
+        S.dfr = P.w.dfr[row];
+        S.dmode = S.dfr.mode;
+    }
+    __syncthreads();
 }
 
 // ---------------------------------------------------------------- span helpers
@@ -2172,36 +2199,52 @@ FIE_DEV bool span_helper(FinSmem& S, const KParams& P, const int row, const int 
 
 // One workgroup per row.  A row's finish is a chain of dependent steps, so its
 // latency is the kernel's: with no more rows than CUs (one workgroup each) the WIDE
-// variant takes up to 256 registers a lane (12 spilled, in the full-row paths); larger
-// batches take 128 (two workgroups a CU).
+// variant takes up to 256 registers a lane and spills none; larger batches take 128 (two
+// workgroups a CU).
 template <int DT, bool WIDE>
 __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KParams P)
 {
     __shared__ FinSmem S;
     if constexpr (WIDE) {
-        // a row the candidates could not settle takes the full-row path here, at once;
-        // with span helpers, in whichever of the row's workgroups arrives last
-        bool deep, inl = true, hd = false;
+        // a row the candidates could not settle takes a full-row path here, at once; with
+        // span helpers, in whichever of the row's workgroups arrives last
+        const int row = blockIdx.x;
+        bool hd = false;
         if (blockIdx.y > 0) {
-            deep = span_helper<DT>(S, P, blockIdx.x, blockIdx.y - 1);
-            inl = false;
+            if (!span_helper<DT>(S, P, row, blockIdx.y - 1)) return;
+            take_row(S, P, row);
             hd = true;
         } else {
-            finish_row<DT, 0, 10, true>(S, P, blockIdx.x, true);
+            finish_row<DT, 10, true>(S, P, row);
             __syncthreads();
-            deep = S.dmode != 0;
-            if (P.helpers && helped_row(P, blockIdx.x)) {
+            if (P.helpers && helped_row(P, row)) {
                 // the record goes out only with a row for the full-row path
-                if (deep && threadIdx.x == 0) P.w.dfr[blockIdx.x] = S.dfr;
-                deep = arrive(S, P, blockIdx.x, deep ? 1u + kArrDeep : 1u, deep) > 0;
+                const bool deep = S.dmode != 0;
+                if (deep && threadIdx.x == 0) P.w.dfr[row] = S.dfr;
+                if (arrive(S, P, row, deep ? 1u + kArrDeep : 1u, deep) <= 0) return;
                 hd = true;
             }
         }
-        if (deep) finish_row<DT, 1, kReloadQ, true>(S, P, blockIdx.x, inl, hd);
+        if (S.dmode == kDeferDraw) {
+            binned_row<DT>(S, P, row, hd);
+            __syncthreads();
+            if (S.dmode == kDeferWindows) {
+                window_row<DT>(S, P, row, true);
+                __syncthreads();
+            }
+        }
+        if (S.dmode != 0) radix_row<DT>(S, P, row);
     } else {
-        finish_row<DT, 0, kReloadQ, false>(S, P, blockIdx.x, false);
+        finish_row<DT, kReloadQ, false>(S, P, blockIdx.x);
         __syncthreads();
-        if (S.dmode == kDeferWindows) window_row<DT>(S, P, blockIdx.x);
+        if (S.dmode != kDeferWindows) return;
+        window_row<DT>(S, P, blockIdx.x, false);
+        __syncthreads();
+        if (S.dmode != 0 && threadIdx.x == 0) {
+            DeferRec d = S.dfr;
+            d.mode = S.dmode;
+            queue_row(P, blockIdx.x, d);
+        }
     }
 }
 
@@ -2215,13 +2258,13 @@ __global__ __launch_bounds__(kFinThreads, 4) void k_deep(const KParams P)
     const uint32_t queued = P.w.dq[0];
     const uint32_t total = queued < (uint32_t)P.a.rows ? queued : (uint32_t)P.a.rows;
     if (blockIdx.x >= total) return;
-    // k_finish launched again on one scan's partials queues its rows again: the first
-    // entry settles a row, for two workgroups would share its list
-    const uint32_t row = P.w.dqrows[blockIdx.x];
-    bool again = false;
-    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kFinThreads) again |= P.w.dqrows[i] == row;
-    if (__syncthreads_or(again)) return;
-    finish_row<DT, 1, kReloadQ, false>(S, P, (int)row, false);
+    const int row = (int)P.w.dqrows[blockIdx.x];
+    take_row(S, P, row);
+    if (S.dmode == kDeferDraw) {
+        binned_row<DT>(S, P, row, false);
+        __syncthreads();
+    }
+    if (S.dmode != 0) radix_row<DT>(S, P, row);
 }
 
 }  // namespace fie

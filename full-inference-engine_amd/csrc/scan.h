@@ -51,16 +51,20 @@ struct RowRes {
     float s;
 };
 
-// A row k_finish hands to k_deep: what the full-row passes need beyond what k_deep
-// recomputes from the partials (mode kDeferDraw), or that the candidates settled
-// the draw and only the top-L logprobs need a pass over the row (kDeferLogprobs).
-// kDeferWindows: the row goes on to window_row in the same workgroup, its mass in tlo and
-// thi, its maximum's bits in token, token 0's key in tau.
-constexpr uint32_t kDeferDraw = 1, kDeferLogprobs = 2, kDeferWindows = 3;
+// A row that goes on to the full-row paths, in the same workgroup or in k_deep: what they
+// need beside the tile table and the row's settings, and what is next: the cut and the
+// draw (by windows, by bins, or by radix levels), or only the top-L logprobs, with the
+// draw settled.
+constexpr uint32_t kDeferDraw = 1, kDeferLogprobs = 2, kDeferWindows = 3, kDeferRadix = 4;
 struct DeferRec {
-    uint64_t tok_comp, cut, tlo, thi;
+    u128 T, sall;            // kept mass; the row's mass
+    uint64_t tok_comp, cut;
     int64_t token;
-    uint32_t tau, mode;
+    uint32_t tau, k0;        // survivors' lowest key; token 0's key
+    float M;                 // the row maximum
+    int32_t status;
+    uint32_t needl;          // its top-L logprobs need a pass over the row
+    uint32_t mode;
 };
 
 // Device pointers into the caller's workspace.
