@@ -305,8 +305,10 @@ FIE_DEV float win_y(float x, float s, float rs)
 //
 // Penalised tokens, token 0 and those past the row read NaN in x[], which every step
 // passes over; the penalised ones follow one a lane, their logits penalised.  Their
-// counts come from k_prep's span bucket, or from the whole history where that
-// overflowed.  The next tile's loads are in flight while one is processed.
+// counts come from k_prep's span bucket, or, where that overflowed, from the whole history,
+// read once for the eight tiles that the waves hold (48 rows of vocab 151936 with 16384 ids
+// 366 us a step, with 60000 750; 1000 and 3560 when each wave read it for its own tile).
+// The next tile's loads are in flight while one is processed.
 enum { kWinCount, kWinSub, kWinWeigh };
 
 // A value that the optimizer does not know to equal v: it would take 32 tokens'
@@ -383,8 +385,11 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
         if (ok && has_cut && c > hi1) m1 += weight_of(S, y, idx);
     };
 
+    constexpr int kGroup = kFinThreads / 64;              // tiles the waves take at a time
+    constexpr int kGroupSpans = kGroup / kWavesPerWG;
+    static_assert(kGroupSpans == 2, "two spans' id counts per group");
     uint4 nxt[NL];
-    uint32_t nnb = 0, nof = 0;
+    uint32_t nnb[kGroupSpans] = {}, nof = 0;
     auto issue = [&](int t) {
         // past the last tile the last one is loaded again, unused: the loads in flight
         // are then the same at every step
@@ -399,12 +404,16 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
         }
         if (pen) {
             const size_t sr = (size_t)row * P.NS + tt / kWavesPerWG;
-            nnb = P.w.nb[sr];
+            // both spans' of the group, so that all waves agree on how to count it
+#pragma unroll
+            for (int k = 0; k < kGroupSpans; ++k)
+                nnb[k] = P.w.nb[(size_t)row * P.NS + min((t - wave) / kWavesPerWG + k, P.NS - 1)];
             nof = P.w.bk[sr * kBucketCap + lane];
         }
     };
     issue(wave);
-    for (int t = wave; t < NT; t += kFinThreads / 64) {
+    for (int t0 = 0; t0 < NT; t0 += kGroup) {
+        const int t = t0 + wave;
         const int lo = t * kTile;
         float x[kEPT];
 #pragma unroll
@@ -412,8 +421,10 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
 #pragma unroll
             for (int e = 0; e < EPL; ++e) x[j * EPL + e] = lane_get<DT>(nxt[j], e);
         }
-        const uint32_t nb = nnb, of = nof;
-        issue(t + kFinThreads / 64);
+        const uint32_t nb = wave < kWavesPerWG ? nnb[0] : nnb[1], of = nof;
+        // the same in every wave: the barriers below depend on it
+        const bool whole = __builtin_amdgcn_readfirstlane((int)max(nnb[0], nnb[1])) > kBucketCap;
+        issue(t + kGroup);
         uint32_t any = 0;
         if (pen) {
             const int sp = t / kWavesPerWG;
@@ -429,15 +440,29 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
                 atomicAdd(&cnt[o >> 1], 1u << ((o & 1) * 16));
                 atomicOr(&bits[o >> 5], 1u << (o & 31));
             };
-            if (nb <= (uint32_t)kBucketCap) {
+            if (whole) {
+                // a span's ids ran past its bucket: all the waves read the whole history once
+                // for their tiles together, four ids a thread in flight
+                __syncthreads();
+                const int64_t h0 = a.hist_offsets[row], h1 = hist_end(a, row);
+                for (int64_t h = h0 + tid; h < h1; h += 4 * kFinThreads) {
+                    uint32_t id[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        id[k] = h + k * kFinThreads < h1 ? (uint32_t)a.hist_ids[h + k * kFinThreads] : 0u;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const uint32_t o = id[k] - (uint32_t)(t0 * kTile);
+                        if (id[k] == 0 || id[k] >= (uint32_t)V || o >= (uint32_t)(kGroup * kTile)) continue;
+                        const uint32_t w = o / kTile, ot = o % kTile;
+                        atomicAdd(&S.tp.cnt[w][ot >> 1], 1u << ((ot & 1) * 16));
+                        atomicOr(&S.tp.bits[w][ot >> 5], 1u << (ot & 31));
+                    }
+                }
+                __syncthreads();
+            } else if (t < NT) {
                 if ((uint32_t)lane < nb) count(of - toff);
                 for (uint32_t i = lane + 64; i < nb; i += 64) count((uint32_t)P.w.bk[sr * kBucketCap + i] - toff);
-            } else {
-                const int64_t h0 = a.hist_offsets[row], h1 = hist_end(a, row);
-                for (int64_t h = h0 + lane; h < h1; h += 64) {
-                    const uint32_t id = (uint32_t)a.hist_ids[h];
-                    if (id != 0 && id < (uint32_t)V) count(id - (uint32_t)lo);
-                }
             }
             wave_lds_sync();
             any = bits[lane];
@@ -454,6 +479,7 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
                                           (__builtin_amdgcn_sbfe((int)mine, (unsigned)i, 1u) & 0x7FC00000));
             }
         }
+        if (t >= NT) continue;                            // past the row: counted with the others, no more
         if (t == 0 && lane == 0) x[0] = __builtin_nanf("");
         if (lo + kTile > V) {
 #pragma unroll

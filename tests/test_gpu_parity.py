@@ -807,3 +807,30 @@ def test_rows_of_batches_past_the_cu_count(fs, dtype):
         torch.cuda.synchronize()
         for key, want in first.items():
             np.testing.assert_array_equal(buf.outputs()[key], want, err_msg=f"{key}, launch {again + 2}")
+
+
+@pytest.mark.parametrize("rows", [20, 300])
+@pytest.mark.parametrize("vocab", [16384, 20011, 51300])
+def test_windowed_rows_with_long_histories(fs, rows, vocab):
+    """Histories of which some spans hold more ids than a bucket (512), so that the eight
+    tiles around are counted from the whole history: in the row's first span, its last (where
+    some waves hold no tile), all of them, none; ids past the vocabulary and token 0 among
+    them."""
+    rng = np.random.default_rng(vocab + rows)
+    x = _deep_rows(rng, rows, vocab, torch.bfloat16, "flat")
+    last = (vocab - 1) // 8192 * 8192
+    params, contexts = [], []
+    for r in range(rows):
+        params.append(SamplingParams(temperature=(1.0, 0.7)[r % 2], top_p=(0.95, 1.0, 0.8)[r % 3],
+                                     repetition_penalty=1.2, presence_penalty=0.1, frequency_penalty=0.02))
+        ids = [rng.integers(0, vocab, 100)]
+        if r % 5 in (1, 3):
+            ids.append(rng.integers(0, min(8192, vocab), 700 + 300 * (r % 2)))
+        if r % 5 in (2, 3):
+            ids.append(rng.integers(last, vocab, 900))
+        if r % 5 == 4:
+            ids.append(rng.integers(0, vocab, 9000))
+        contexts.append(np.concatenate(ids + [[0, vocab - 1, vocab - 1]]).tolist())
+    out, ref, _, _ = run_both(fs, x, params, rng.random(rows), contexts, kept=False)
+    check(out, ref, params)
+    assert ((out["status"] & _lib.FIE_ROW_EXACT_PATH) != 0).sum() > rows // 2
