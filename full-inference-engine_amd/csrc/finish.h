@@ -1371,6 +1371,14 @@ FIE_DEV float row_logprob(uint64_t comp, float M, double lse)
     return (float)(((double)key_to_float(comp_k(comp)) - (double)M) - lse);
 }
 
+// Rows of at most this many tiles take the bins instead of the windows, whose passes give
+// a wave a tile: with most of the waves idle the block-wide passes are faster.  us a step,
+// bins against windows (20 flat rows / 1024 / 48 open ones with 2000 ids): 2 tiles 55 / 120 /
+// 78 against 65 / 210 / 94, 4 tiles 57 / 135 / 86 against 64 / 154 / 91, 6 tiles 63 / 157 / 98
+// against 67 / 171 / 97, 7 tiles 66 / 166 / 102 against 67 / 176 / 95, 8 tiles 68 / 175 / 105
+// against 65 / 174 / 90.
+constexpr int kBinTiles = 3 * (kFinThreads / 64) / 4;
+
 // Whether no threshold restricts a sampled row but its top-p cut.
 FIE_DEV bool plain_cut(int topk, float mp) { return topk == 0 && !(mp > 0.0f); }
 
@@ -1733,22 +1741,7 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row)
     // settle.)
     uint32_t next = 0;
     if (deep) {
-        const bool plain = plain_cut(topk, mp);
-        next = plain && !P.helpers ? kDeferWindows : kDeferDraw;
-        if constexpr (WIDE) {
-            if (next == kDeferWindows) {
-                // the list may run on into the candidate slots unless the logprobs read them again
-                const WinList list{P.w.cand + (size_t)row * NT * kCapW, (uint32_t)(kGCap + (lp > 0 ? 0 : NT * kCapW))};
-                next = kDeferDraw;
-                if (windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, list, &cut, &T, &tok_comp)) {
-                    next = 0;
-                    status |= FIE_ROW_EXACT_PATH;
-                    tau = 0;
-                    token = comp_idx(tok_comp);
-                    if (a.tk_key && tid == 0) a.tk_key[row] = 0;
-                }
-            }
-        }
+        next = plain_cut(topk, mp) && !P.helpers && NT > kBinTiles ? kDeferWindows : kDeferDraw;
         // the LDS candidates again, for the logprobs
         sorted = false;
         if (lp > 0) {
@@ -1779,6 +1772,20 @@ FIE_DEV void finish_row(FinSmem& S, const KParams& P, const int row)
         }
     }
 
+    if constexpr (WIDE) {
+        if (next == kDeferWindows) {
+            const WinList list{P.w.cand + (size_t)row * NT * kCapW, (uint32_t)(kGCap + NT * kCapW)};
+            next = kDeferDraw;
+            if (windowed_deep<DT>(S, P, row, s, pen, rep, pres, freq, k0, M, tp, urow, sall, list, &cut, &T, &tok_comp)) {
+                next = 0;
+                status |= FIE_ROW_EXACT_PATH;
+                tau = 0;
+                token = comp_idx(tok_comp);
+                if (tid == 0 && a.tk_key) a.tk_key[row] = 0;
+                if (tid == 0 && lp >= 0 && a.chosen_logprob) a.chosen_logprob[row] = row_logprob(tok_comp, M, lse);
+            }
+        }
+    }
     if (tid != 0) return;
     if (next == 0 && !needl) {
         write_row(P, row, token, status, M, cut, T, sall, tau, greedy, s);

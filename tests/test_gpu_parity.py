@@ -618,7 +618,7 @@ def test_span_helpers_lone_rows_and_odd_shapes(fs):
     z[:, 0] = 6.0                                             # token 0 is the maximum
     params = [SamplingParams(temperature=1.0, top_p=0.999), SamplingParams(temperature=1.0)]
     out, ref, gk, gp = run_both(fs, z, params, np.array([0.999, 0.999]))
-    assert (out["status"] & _lib.FIE_ROW_EXACT_PATH).all()
+    assert ((out["status"] & _lib.FIE_ROW_EXACT_PATH) != 0).sum() > rows * 3 // 4
     check(out, ref, params, gk, gp)
 
 
@@ -834,3 +834,21 @@ def test_windowed_rows_with_long_histories(fs, rows, vocab):
     out, ref, _, _ = run_both(fs, x, params, rng.random(rows), contexts, kept=False)
     check(out, ref, params)
     assert ((out["status"] & _lib.FIE_ROW_EXACT_PATH) != 0).sum() > rows // 2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,vocab", [(20, 300), (20, 2049), (20, 12288), (20, 12289), (300, 4001), (300, 12288), (300, 12289)])
+def test_short_rows_on_both_sides_of_the_windows(fs, dtype, rows, vocab):
+    """Deep rows of up to six tiles take the bins, of seven and more the windows: the same
+    answers as the oracle on both sides, penalised (a history that overflows its span's bucket
+    among them) or not, with logprobs, and with thresholds below the candidates."""
+    rng = np.random.default_rng(vocab)
+    x = torch.cat([_deep_rows(rng, rows // 2, vocab, dtype, kind) for kind in ("flat", "grid")])
+    pen = dict(repetition_penalty=1.3, frequency_penalty=0.05, presence_penalty=0.2)
+    kinds = [dict(temperature=1.0, top_p=0.95), dict(temperature=1.0, top_p=0.9, **pen), dict(temperature=0.8),
+             dict(temperature=1.2, logprobs=8, **pen), dict(temperature=1.0, top_p=0.99, logprobs=0),
+             dict(temperature=1.0, min_p=0.4, **pen), dict(temperature=1.0, top_k=3000, top_p=0.9, **pen)]
+    params = [SamplingParams(**kinds[r % len(kinds)]) for r in range(rows)]
+    ctx = [rng.integers(0, vocab, 50 if r % 2 else 1500).tolist() for r in range(rows)]
+    out, ref, gk, gp = run_both(fs, x, params, rng.random(rows), ctx)
+    check(out, ref, params, gk, gp, lp=True)
