@@ -852,3 +852,28 @@ def test_short_rows_on_both_sides_of_the_windows(fs, dtype, rows, vocab):
     ctx = [rng.integers(0, vocab, 50 if r % 2 else 1500).tolist() for r in range(rows)]
     out, ref, gk, gp = run_both(fs, x, params, rng.random(rows), ctx)
     check(out, ref, params, gk, gp, lp=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [24, 280])
+def test_penalised_thresholds_below_the_candidates(fs, dtype, rows):
+    """Penalised rows with a top-k or min-p threshold below their candidates take the binned
+    passes and the radix levels, past the helper limit and past the CU count: spans whose
+    buckets hold the counts (both of a span's chunks), spans that overflow theirs, an odd
+    vocabulary, 16-bit logits that share values."""
+    rng = np.random.default_rng(rows)
+    vocab = 30001
+    x = torch.cat([_deep_rows(rng, rows // 2, vocab, dtype, kind) for kind in ("flat", "grid")])
+    pen = dict(repetition_penalty=1.3, frequency_penalty=0.05, presence_penalty=0.2)
+    kinds = [dict(temperature=1.0, top_k=3000, top_p=0.9, **pen), dict(temperature=1.0, min_p=0.3, **pen),
+             dict(temperature=1.1, top_k=6000, **pen), dict(temperature=1.0, min_p=0.2, top_k=2500, top_p=0.8, **pen)]
+    params = [SamplingParams(**kinds[r % len(kinds)]) for r in range(rows)]
+    ctx = []
+    for r in range(rows):
+        ids = [rng.integers(0, vocab, 400), rng.integers(4096, 8192, 40), [0]]
+        if r % 3 == 1:
+            ids.append(rng.integers(8192, 16384, 800))
+        ctx.append(np.concatenate(ids).tolist())
+    out, ref, _, _ = run_both(fs, x, params, rng.random(rows), ctx, kept=False)
+    check(out, ref, params)
+    assert ((out["status"] & _lib.FIE_ROW_EXACT_PATH) != 0).sum() > rows * 3 // 4
