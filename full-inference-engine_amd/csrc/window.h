@@ -24,12 +24,13 @@ namespace fie {
 // Bins of the count: the top bits of the float d + 1, so 2^kWinOct bins to each
 // octave: 1/512 wide at the row's maximum, 1/32 at d = 31, past which every share of
 // the mass is below e^-31.  Bin 0 takes what rounding pushes below d = 0.  A bin holds
-// its tokens' count (high word) and the sum of the kWinShift bits of d + 1 below the
-// bin's own, so that its mass is taken at its tokens' mean d: 16-bit logits put
-// thousands of tokens at one place in a bin, and taking its middle was off by 10^-3
-// of the row's mass.
+// its tokens' count (high word) and the sum of the kWinSubs bits of d + 1 below the
+// bin's own (all but the last one: a bin may hold every token of the row), so that its
+// mass is taken at its tokens' mean d: 16-bit logits put thousands of tokens at one place
+// in a bin, and taking its middle was off by 10^-3 of the row's mass.
 constexpr int kWinOct = 9, kWinOctaves = 5;
-constexpr int kWinShift = 23 - kWinOct;
+constexpr int kWinShift = 23 - kWinOct, kWinSubs = kWinShift - 1;
+static_assert((uint64_t)kMaxTiles * kTile * ((1u << kWinSubs) - 1) < 1ull << 32, "a bin's sum stays in its word");
 constexpr uint32_t kWinOrg = (0x3F800000u >> kWinShift) - 1;
 constexpr int kWinBins = kWinOctaves * (1 << kWinOct) + 1;
 // What is added to d: one, and a shift that keeps the bins' edges off the multiples of
@@ -68,7 +69,7 @@ FIE_DEV float win_mass(const FinSmem& S, const Win& w, int k, int j, float M)
     if (c == 0) return 0.0f;
     float y;
     if (k < 0) {
-        const uint32_t mean = (uint32_t)((float)(uint32_t)S.cand[j] / (float)c);
+        const uint32_t mean = (uint32_t)(2.0f * ((float)(uint32_t)S.cand[j] / (float)c));
         y = kWinOne - __uint_as_float(((uint32_t)(j + (int)kWinOrg) << kWinShift) + mean);
         return (float)c * __expf(y);
     }
@@ -349,7 +350,7 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
         const uint32_t f = __float_as_uint(__builtin_fmaf(x, -rs, off));
         const uint32_t b = (f >> kWinShift) - kWinOrg;
         if (ok && b < (uint32_t)kWinBins)
-            atomicAdd((unsigned long long*)&S.cand[b], (1ull << 32) | (f & ((1u << kWinShift) - 1)));
+            atomicAdd((unsigned long long*)&S.cand[b], (1ull << 32) | ((f >> 1) & ((1u << kWinSubs) - 1)));
     };
     // a window's token in a refining count
     uint32_t kmin[2] = {0xFFFFFFFFu, 0xFFFFFFFFu}, kmax[2] = {0, 0};

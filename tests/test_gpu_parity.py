@@ -877,3 +877,47 @@ def test_penalised_thresholds_below_the_candidates(fs, dtype, rows):
     out, ref, _, _ = run_both(fs, x, params, rng.random(rows), ctx, kept=False)
     check(out, ref, params)
     assert ((out["status"] & _lib.FIE_ROW_EXACT_PATH) != 0).sum() > rows * 3 // 4
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_windowed_rows_of_the_largest_vocabulary(fs, dtype):
+    """524288 tokens, three quarters of them or all at one value (one bin of the count), and
+    rows that mask most tokens with -inf or the type's lowest value."""
+    vocab, rows = 524288, 20
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(rows, vocab, generator=g)
+    x[:8, vocab // 4:] = -6.2
+    x[8:10] = 0.7
+    x[10:14, vocab // 3:] = float("-inf")
+    x[14:16, 5000:] = torch.finfo(dtype).min
+    x = x.to(dtype)
+    params = [SamplingParams(temperature=(1.0, 1.3)[r % 2], top_p=(1.0, 0.97, 0.9)[r % 3],
+                             presence_penalty=0.3 * (r % 4 == 3)) for r in range(rows)]
+    ctx = [torch.randint(0, vocab, (300,), generator=g).tolist() for _ in range(rows)]
+    u = np.linspace(0.02, 0.98, rows)
+    out, ref, _, _ = run_both(fs, x, params, u, ctx, kept=False)
+    check(out, ref, params)
+    assert ((out["status"] & _lib.FIE_ROW_EXACT_PATH) != 0).sum() > rows // 2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [20, 300])
+def test_windowed_rows_with_masked_tokens_and_large_maxima(fs, dtype, rows):
+    """Rows with banned tokens (-inf, which the fp16 passes see as NaN, or the type's lowest
+    value), with half of them, and rows whose maximum is too large for the count's bins."""
+    vocab = 20480 + 77
+    rng = np.random.default_rng(rows)
+    x = _deep_rows(rng, rows, vocab, dtype, "flat").float()
+    ban = torch.from_numpy(rng.random((rows, vocab)) < np.where(np.arange(rows) % 2, 0.5, 0.01)[:, None])
+    ban[:, 7] = False
+    low = torch.where(torch.arange(rows) % 4 < 2, float("-inf"), float(torch.finfo(dtype).min))
+    x = torch.where(ban, low[:, None], x)
+    big = torch.arange(rows) % 5 == 4
+    x[big] += {torch.float32: 2.0 ** 25, torch.bfloat16: 2.0 ** 25, torch.float16: 30000.0}[dtype]
+    x = x.to(dtype)
+    params = [SamplingParams(temperature=(1.0, 0.8)[r % 2], top_p=(0.95, 1.0, 0.7)[r % 3],
+                             repetition_penalty=1.1 if r % 7 == 3 else 1.0) for r in range(rows)]
+    ctx = [rng.integers(0, vocab, 200).tolist() for _ in range(rows)]
+    out, ref, _, _ = run_both(fs, x, params, rng.random(rows), ctx, kept=False)
+    check(out, ref, params)
+    assert ((out["status"] & _lib.FIE_ROW_EXACT_PATH) != 0).sum() > rows // 2
