@@ -275,30 +275,11 @@ FIE_DEV uint64_t shfl_xor_u64(uint64_t v, int m)
     return ((uint64_t)hi << 32) | lo;
 }
 
-FIE_DEV uint64_t shfl_up_u64(uint64_t v, int d)
-{
-    uint32_t lo = __shfl_up((uint32_t)v, d, 64);
-    uint32_t hi = __shfl_up((uint32_t)(v >> 32), d, 64);
-    return ((uint64_t)hi << 32) | lo;
-}
-
 FIE_DEV uint64_t shfl_u64(uint64_t v, int src)
 {
     uint32_t lo = __shfl((uint32_t)v, src, 64);
     uint32_t hi = __shfl((uint32_t)(v >> 32), src, 64);
     return ((uint64_t)hi << 32) | lo;
-}
-
-FIE_DEV u128 shfl_up_u128(u128 v, int d)
-{
-    uint64_t lo = shfl_up_u64((uint64_t)v, d), hi = shfl_up_u64((uint64_t)(v >> 64), d);
-    return ((u128)hi << 64) | lo;
-}
-
-FIE_DEV u128 shfl_xor_u128(u128 v, int m)
-{
-    uint64_t lo = shfl_xor_u64((uint64_t)v, m), hi = shfl_xor_u64((uint64_t)(v >> 64), m);
-    return ((u128)hi << 64) | lo;
 }
 
 FIE_DEV uint32_t wave_max_u32(uint32_t v)
@@ -340,28 +321,12 @@ FIE_DEV uint64_t wave_sum_u64(uint64_t v)
     return v;
 }
 
-FIE_DEV u128 wave_sum_u128(u128 v)
-{
-    for (int m = 32; m > 0; m >>= 1) v += shfl_xor_u128(v, m);
-    return v;
-}
-
 // Inclusive prefix sum over the lanes of a wave (lane 0 first).
 FIE_DEV uint32_t wave_incl_scan_u32(uint32_t v)
 {
     const int lane = threadIdx.x & 63;
     for (int d = 1; d < 64; d <<= 1) {
         uint32_t o = __shfl_up(v, d, 64);
-        if (lane >= d) v += o;
-    }
-    return v;
-}
-
-FIE_DEV u128 wave_incl_scan_u128(u128 v)
-{
-    const int lane = threadIdx.x & 63;
-    for (int d = 1; d < 64; d <<= 1) {
-        u128 o = shfl_up_u128(v, d);
         if (lane >= d) v += o;
     }
     return v;

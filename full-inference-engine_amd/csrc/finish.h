@@ -128,7 +128,7 @@ struct Pred {
 // MASS) first exceeds g: excl <= g < excl + meas.  Digits are 8-bit windows placed
 // just below the common prefix of the remaining range, so few levels are needed.
 template <bool MASS>
-FIE_DEV SelResult lds_select(FinSmem& S, const uint64_t* cand, int n, const Pred pr, u128 g)
+FIE_DEV SelResult lds_select(FinSmem& S, int n, const Pred pr, u128 g)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint64_t prefix = 0, pmask = 0;
@@ -137,7 +137,7 @@ FIE_DEV SelResult lds_select(FinSmem& S, const uint64_t* cand, int n, const Pred
         // range of the remaining elements (one barrier), and a cleared histogram
         uint64_t mn = ~0ull, mx = 0;
         for (int i = tid; i < n; i += kFinThreads) {
-            const uint64_t c = cand[i];
+            const uint64_t c = S.cand[i];
             if ((c & pmask) == prefix && pr(c)) {
                 mn = c < mn ? c : mn;
                 mx = c > mx ? c : mx;
@@ -168,7 +168,7 @@ FIE_DEV SelResult lds_select(FinSmem& S, const uint64_t* cand, int n, const Pred
         const int shift = hb >= 7 ? hb - 7 : 0;
         const uint64_t hmask = (hb >= 63) ? 0ull : ~((2ull << hb) - 1);
         for (int i = tid; i < n; i += kFinThreads) {
-            const uint64_t c = cand[i];
+            const uint64_t c = S.cand[i];
             if ((c & pmask) == prefix && pr(c)) {
                 const int d = (int)((c >> shift) & 0xFFu);
                 if (MASS) {
@@ -432,7 +432,7 @@ FIE_DEV SelResult row_select(FinSmem& S, const KParams& P, int row, float s, boo
         if (cnt <= (uint32_t)kGCap) {
             const int n = pass_gather<DT>(S, P, row, s, pen, rep, pres, freq, k0, pr,
                                                dg.shift, hiprefix);
-            SelResult r = lds_select<MASS>(S, S.cand, n, pr, g);
+            SelResult r = lds_select<MASS>(S, n, pr, g);
             r.excl += excl;
             return r;
         }
@@ -702,7 +702,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
         u128 above;
         const int b = dbin_pick<false>(S, kPassBins - 1, (u128)S.pc[kPassBins - 1], (u128)(topk - 1), &above);
         if (b < 0 || !gather(b, b)) return false;
-        const SelResult r = lds_select<false>(S, S.cand, ncur, Pred{0, 0, 0}, (u128)(topk - 1) - above);
+        const SelResult r = lds_select<false>(S, ncur, Pred{0, 0, 0}, (u128)(topk - 1) - above);
         if (!r.found) return false;
         tk = comp_k(r.comp);
     }
@@ -765,7 +765,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
             }
             Pred pc{tau, 0, 0};
             pc.hi = chi;
-            const SelResult r = lds_select<true>(S, S.cand, ncur, pc, thr - 1 - above);
+            const SelResult r = lds_select<true>(S, ncur, pc, thr - 1 - above);
             if (!r.found) return false;
             cut = r.comp;
             T = above + r.excl + r.meas;
@@ -780,7 +780,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
         u128 above;
         const int b = dbin_pick<false>(S, kPassBins - 1, (u128)S.pc[kPassBins - 1], 0, &above);
         if (b < 0 || !gather(b, b)) return false;
-        const SelResult r = lds_select<false>(S, S.cand, ncur, Pred{0, 0, 0}, 0);
+        const SelResult r = lds_select<false>(S, ncur, Pred{0, 0, 0}, 0);
         if (!r.found) return false;
         tok = r.comp;
     } else {
@@ -807,7 +807,7 @@ FIE_DEV bool binned_deep(FinSmem& S, const KParams& P, int row, float s, bool pe
                 pd.hi = mn - 1;
             }
         }
-        const SelResult r = lds_select<true>(S, S.cand, ncur, pd, g - base);
+        const SelResult r = lds_select<true>(S, ncur, pd, g - base);
         if (!r.found) return false;
         tok = r.comp;
     }

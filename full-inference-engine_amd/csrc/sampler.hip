@@ -241,7 +241,7 @@ static bool layout_of(int32_t R, int32_t V, Layout* L)
     L->res = take(r * sizeof(RowRes));
     L->mt = take(r * (NT + 1) * 4);
     L->ct = take(r * (NT + 1) * 8);
-    L->dq = take(2 * 4);
+    L->dq = take(4);
     L->dqrows = take(r * 4);
     L->dfr = take(r * sizeof(DeferRec));
     // span helpers of k_finish: only workspaces for at most kHelpRows rows hold them

@@ -83,7 +83,7 @@ struct Ws {
     RowRes* res;         // [rows]
     float* mt;           // [rows * (NT + 1)] tile maxima of y, slot 0 = token 0
     uint64_t* ct;        // [rows * (NT + 1)] tile scales C_t
-    uint32_t* dq;        // [2] rows queued for k_deep, and taken; k_scan clears both
+    uint32_t* dq;        // [1] rows queued for k_deep; k_scan clears it
     uint32_t* dqrows;    // [rows] the queued rows
     DeferRec* dfr;       // [rows]
     // Span helpers of k_finish (batches of at most kHelpRows rows; NULL otherwise),
@@ -659,7 +659,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(const KParams P)
     const bool pen = rc.pen;
     const char* rowp = (const char*)a.logits + (size_t)row * (size_t)a.row_stride * SZ;
     const size_t slot = (size_t)row * NT + tile;
-    if (blockIdx.x == 0 && blockIdx.y == 0 && tid < 2) P.w.dq[tid] = 0u;   // k_deep's queue, filled by k_finish
+    if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) P.w.dq[0] = 0u;    // k_deep's queue, filled by k_finish
     if (P.helpers && blockIdx.x == 0 && tid == 0) P.w.harr[row] = 0u;     // k_finish's arrivals at the row
 
     // 1. The span's history bucket (k_prep), then every load of the tile: the

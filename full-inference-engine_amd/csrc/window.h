@@ -338,10 +338,6 @@ FIE_DEV void win_pass(FinSmem& S, const KParams& P, int row, int phase, float s,
     const float rs = 1.0f / s, off = M + kWinOne;
     const uint32_t use = phase == kWinSub ? S.wbig : (has_cut ? 3u : 1u);      // the windows looked at
 
-    auto uni64 = [](uint64_t v) {
-        return ((uint64_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-    };
     const uint64_t lo0 = uni64(S.win[0].lo), hi0 = uni64(S.win[0].hi);
     const uint64_t lo1 = uni64(S.win[1].lo), hi1 = uni64(S.win[1].hi);
 

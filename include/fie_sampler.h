@@ -172,9 +172,13 @@ int fie_sampler_lmhead_stage(const fie_sampler_args* args, const void* hidden, c
 enum {
     FIE_STAGE_PREP = 0,        /* the penalty histories bucketed by span (no-op without penalties) */
     FIE_STAGE_SCAN = 1,        /* the streaming pass over the logits */
-    FIE_STAGE_FINISH = 2,      /* the per-row selection and draw from the candidates */
-    FIE_STAGE_DEEP = 3,        /* the rows FINISH queued: passes over the whole row (no-op when none;
-                                  FINISH queues none when rows <= the GPU's CUs) */
+    FIE_STAGE_FINISH = 2,      /* the per-row selection and draw: from the candidates, or over the
+                                  whole row.  Launched again after one SCAN it gives the same
+                                  outputs, but may take longer: it uses the candidate slots of
+                                  rows it takes through the whole row */
+    FIE_STAGE_DEEP = 3,        /* the rows FINISH queued: thresholds or logprobs below the
+                                  candidates, and whole rows that FINISH does not take (no-op when
+                                  none; FINISH queues none when rows <= the GPU's CUs) */
 };
 int fie_sampler_stage(const fie_sampler_args* args, const fie_workspace* ws, int32_t stage,
                       void* stream);
