@@ -2224,9 +2224,10 @@ __global__ __launch_bounds__(kFinThreads, WIDE ? 2 : 4) void k_finish(const KPar
         } else {
             finish_row<DT, 10, true>(S, P, row);
             __syncthreads();
+            const bool deep = S.dmode != 0;
+            if (__builtin_expect(!deep && !P.helpers, 1)) return;
             if (P.helpers && helped_row(P, row)) {
                 // the record goes out only with a row for the full-row path
-                const bool deep = S.dmode != 0;
                 if (deep && threadIdx.x == 0) P.w.dfr[row] = S.dfr;
                 if (arrive(S, P, row, deep ? 1u + kArrDeep : 1u, deep) <= 0) return;
                 hd = true;
